@@ -444,57 +444,17 @@ struct PrefillArgs {
     float* z;                // split-K output: partial sums [mats][sk][P][N] fp32 (no epilogue)
 };
 
-// The A fragment of one 16-column trellis tile over two k tiles (K = 4): lane l owns column c = l % 16 of the tile
-// (format lane i = c % 8, value half c / 8) for k tile q / 2 and word pair g = q % 2 (q = l / 16): words 4i + 2g and
-// 4i + 2g + 1 hold its 8 values, rows (2l + 8 + h, 2l + h) for l = 2g, 2g + 1 -- the pair order of pair_row, the order
-// the token rows are staged in. tw: the tile's words of the two k tiles in LDS, [2][32].
-// The words of that fragment: the previous word and the lane's word pair of its k tile.
-__device__ __forceinline__ void frag4_words(const uint32_t* tw, int lane, uint32_t& p0, uint32_t& w0, uint32_t& w1) {
-    const int c = lane & 15, i = c & 7, q = lane >> 4, kt = q >> 1, g = q & 1;
-    const uint32_t* w = tw + kt * 32;
-    const int w0i = 4 * i + 2 * g;
-    p0 = w[(w0i + 31) & 31];
-    const uint2 ww = *reinterpret_cast<const uint2*>(w + w0i);
-    w0 = ww.x;
-    w1 = ww.y;
-}
-// Its four packed state pairs (each two 16-bit windows of one column, pair order).
-__device__ __forceinline__ void frag4_states(uint32_t p0, uint32_t w0, uint32_t w1, int lane, uint32_t (&s)[4]) {
-    const uint32_t sel = ((lane & 15) >> 3) ? 0x02010100u : 0x04030302u;   // value half: (s6,s4)/(s7,s5) or (s2,s0)/(s3,s1)
-    {
-        const uint32_t a = __builtin_amdgcn_alignbit(p0, w0, 4), b = p0 >> 4;
-        s[0] = __builtin_amdgcn_perm(b, a, sel);
-        s[1] = __builtin_amdgcn_perm(p0, w0, sel);
-    }
-    {
-        const uint32_t a = __builtin_amdgcn_alignbit(w0, w1, 4), b = w0 >> 4;
-        s[2] = __builtin_amdgcn_perm(b, a, sel);
-        s[3] = __builtin_amdgcn_perm(w0, w1, sel);
-    }
-}
-__device__ __forceinline__ h8_t a_fragment4(const uint32_t* tw, int lane) {
-    uint32_t p0, w0, w1, s[4];
-    frag4_words(tw, lane, p0, w0, w1);
-    frag4_states(p0, w0, w1, lane, s);
-    h8_t f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const h2_t v = decode_pair(s[j]);
-        f[2 * j] = v[0];
-        f[2 * j + 1] = v[1];
-    }
-    return f;
-}
-
-// The same fragment for K = 2, 3 and 5 (the prefill path stages its rows in the K != 2 pair order of pair_row at
-// every width). The lane's two value
-// groups (l = 2g and 2g + 1) are each 4 consecutive values 8 l + 4 half .. + 3 of format lane i; their windows end
-// at bits (v + 1) K of the lane's stream and span 3 K + 16 <= 31 bits, so one funnel shift of two adjacent words
-// (alignbit by a per-lane amount, the same for every tile) holds all four: value v0 + d at bits (3 - d) K.
-// fragk_words: the 2 x 2 words of the lane's groups (the word before the group's last bit wraps within the k tile,
-// as lane 0's previous word is lane 7's last); fragk_shifts: the two funnel shifts.
+// The A fragment of one 16-column trellis tile over two k tiles: lane l owns column c = l % 16 of the tile (format lane
+// i = c % 8, value half c / 8) for k tile q / 2 and word group g = q % 2 (q = l / 16). Its 8 values are rows
+// (2l + 8 + h, 2l + h) for l = 2g, 2g + 1 -- the pair order of pair_row (K != 2), the order the token rows are staged
+// in. The two groups (l = 2g and 2g + 1) are each 4 consecutive values 8 l + 4 half .. + 3 of format lane i; their
+// windows end at bits (v + 1) K of the lane's stream and span 3 K + 16 <= 31 bits, so one funnel shift of two adjacent
+// words (alignbit by a per-lane amount, the same for every tile) holds all four: value v0 + d at bits (3 - d) K.
+// frag_words: the 2 x 2 words of the lane's groups from the tile's words of the two k tiles in LDS, [2][8 K] (the word
+// before the group's last bit wraps within the k tile, as lane 0's previous word is lane 7's last); frag_shifts: the
+// two funnel shifts.
 template <int K>
-__device__ __forceinline__ void fragk_groups(int lane, int t, int& lo, int& sh) {
+__device__ __forceinline__ void frag_groups(int lane, int t, int& lo, int& sh) {
     const int c = lane & 15, half = c >> 3, g = (lane >> 4) & 1, i = c & 7;
     const int v0 = 8 * (2 * g + t) + 4 * half;
     const int e = (v0 + 4) * K, hiw = (e - 1) >> 5;
@@ -502,47 +462,87 @@ __device__ __forceinline__ void fragk_groups(int lane, int t, int& lo, int& sh) 
     sh = 32 * (hiw + 1) - e;
 }
 template <int K>
-__device__ __forceinline__ void fragk_shifts(int lane, uint32_t (&sh)[2]) {
+__device__ __forceinline__ void frag_shifts(int lane, uint32_t (&sh)[2]) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         int lo, s;
-        fragk_groups<K>(lane, t, lo, s);
+        frag_groups<K>(lane, t, lo, s);
         sh[t] = (uint32_t)s;
     }
 }
 template <int K>
-__device__ __forceinline__ void fragk_words(const uint32_t* tw, int lane, uint32_t (&wd)[4]) {
+__device__ __forceinline__ void frag_words(const uint32_t* tw, int lane, uint32_t (&wd)[4]) {
     const uint32_t* w = tw + (lane >> 5) * (8 * K);     // k tile q / 2
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    if constexpr (K == 4) {
+        // the groups' words are an aligned pair and the one before it
         int lo, s;
-        fragk_groups<K>(lane, t, lo, s);
-        wd[2 * t] = w[(lo + 8 * K - 1) % (8 * K)];
-        wd[2 * t + 1] = w[lo];
-    }
-}
-// Its four packed state pairs, st[2 t + h] = (window of v0 + h + 2 low, window of v0 + h high).
-template <int K>
-__device__ __forceinline__ void fragk_states(const uint32_t (&wd)[4], const uint32_t (&sh)[2], uint32_t (&st)[4]) {
-    static_assert(3 * K + 16 <= 32, "four windows in one funnel word");
+        frag_groups<4>(lane, 0, lo, s);
+        const uint2 ww = *reinterpret_cast<const uint2*>(w + lo);
+        wd[0] = w[(lo + 31) & 31];
+        wd[1] = wd[2] = ww.x;
+        wd[3] = ww.y;
+    } else {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const uint32_t W = __builtin_amdgcn_alignbit(wd[2 * t], wd[2 * t + 1], sh[t]);
-        st[2 * t] = ((W << (16 - 3 * K)) & 0xFFFF0000u) | ((W >> K) & 0xFFFFu);
-        st[2 * t + 1] = ((W << (16 - 2 * K)) & 0xFFFF0000u) | (W & 0xFFFFu);
+        for (int t = 0; t < 2; ++t) {
+            int lo, s;
+            frag_groups<K>(lane, t, lo, s);
+            wd[2 * t] = w[(lo + 8 * K - 1) % (8 * K)];
+            wd[2 * t + 1] = w[lo];
+        }
     }
 }
+// The lane's 8 weights from its two groups' funnel words: word W of group t holds the four windows v0 + d (d = 0..3) at
+// bits (3 - d) K. Pair j = 2 t + h of the fragment is (window v0 + h + 2 low, window v0 + h high). A window is cut out
+// (v_bfe_u32, or v_and_b32 for the one at bit 0), times the codebook multiplier mod 2^32 (v_mul_lo_u32), mask and
+// flip (v_bitop3), and the two fp16 halves of each word are added straight into their half of the pair
+// (v_add_f16_sdwa: the reference's rounding of lo + hi): 4.25 VALU instructions a weight, where packing two states
+// first (v_perm, two 24-bit multiplies, two v_perm, v_pk_mad_u16, two v_bitop3, v_pk_add_f16) takes 5.1 at K = 4 and
+// 5.75 at K = 3 and 5. Issue cost by instruction (two waves a SIMD): v_and, v_bitop3 with VGPR constants 1.1-1.2 ns;
+// v_bfe, v_alignbit, v_mul_lo_u32, v_add_f16_sdwa 1.9 ns. Same bits as before; measured a layer, before and after (the
+// windows of few rows an expert are bound by this decode): 77 rows, hidden 5120, K = 3 651 -> 515 us; 709 rows, hidden
+// 5120, K = 5 1309 -> 1178 us; 32 rows, hidden 2048, K = 4 100.4 -> 91.1 us; 8192 rows, hidden 2048, K = 4 1191 -> 1182 us.
+struct FragConsts {
+    uint32_t lo16, mask, flip;
+};
+__device__ __forceinline__ FragConsts frag_consts() {
+    FragConsts c{0xffffu, 0x8FFF8FFFu, 0x3B603B60u};
+    __asm__ volatile("" : "+v"(c.lo16), "+v"(c.mask), "+v"(c.flip));   // kept in VGPRs (see above)
+    return c;
+}
+template <int K, int D>
+__device__ __forceinline__ uint32_t frag_codeword(uint32_t W, const FragConsts& c) {
+    const uint32_t s = D == 3 ? (W & c.lo16) : __builtin_amdgcn_ubfe(W, (3 - D) * K, 16);
+    return mask_flip(s * 0xCBAC1FEDu, c.mask, c.flip);
+}
+// (fp16(a.lo + a.hi) low, fp16(b.lo + b.hi) high)
+__device__ __forceinline__ uint32_t halves_sums(uint32_t a, uint32_t b) {
+    uint32_t d;
+    __asm__("v_add_f16_sdwa %0, %1, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+            "v_add_f16_sdwa %0, %2, %2 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
+            : "=&v"(d) : "v"(a), "v"(b));
+    return d;
+}
+template <int K, int H>
+__device__ __forceinline__ h2_t frag_pair(uint32_t W, const FragConsts& c) {
+    return bits_h2(halves_sums(frag_codeword<K, H + 2>(W, c), frag_codeword<K, H>(W, c)));
+}
+// The lane's funnel words of a fragment from its staged words (K = 4: previous word, word pair).
 template <int K>
-__device__ __forceinline__ h8_t a_fragmentk(const uint32_t* tw, int lane, const uint32_t (&sh)[2]) {
-    uint32_t wd[4], s[4];
-    fragk_words<K>(tw, lane, wd);
-    fragk_states<K>(wd, sh, s);
+__device__ __forceinline__ void frag_funnel(const uint32_t (&wd)[4], const uint32_t (&sh)[2], uint32_t (&W)[2]) {
+    static_assert(3 * K + 16 <= 32, "four windows in one funnel word");
+    W[0] = __builtin_amdgcn_alignbit(wd[0], wd[1], sh[0]);
+    W[1] = __builtin_amdgcn_alignbit(wd[2], wd[3], sh[1]);
+}
+template <int K>
+__device__ __forceinline__ h8_t a_fragment(const uint32_t (&wd)[4], const uint32_t (&sh)[2], const FragConsts& c) {
+    uint32_t W[2];
+    frag_funnel<K>(wd, sh, W);
     h8_t f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const h2_t v = decode_pair(s[j]);
-        f[2 * j] = v[0];
-        f[2 * j + 1] = v[1];
+    for (int t = 0; t < 2; ++t) {
+        const h2_t v0 = frag_pair<K, 0>(W[t], c), v1 = frag_pair<K, 1>(W[t], c);
+        f[4 * t] = v0[0]; f[4 * t + 1] = v0[1];
+        f[4 * t + 2] = v1[0]; f[4 * t + 3] = v1[1];
     }
     return f;
 }
@@ -716,17 +716,17 @@ __global__ void __launch_bounds__(256, BM == 256 ? 1 : 2) prefill_gemm_kernel(co
         const int row = 16 * b + (lane & 15);
         return *reinterpret_cast<const h8_t*>(xb + row * 64 + ((q ^ ((row >> 1) & 3)) << 4));
     };
-    // K = 3, 5: the direct fragment decode's two per-lane funnel shifts (the same for every tile and step)
-    uint32_t ksh[2] = {0u, 0u};
-    if constexpr (K != 4) fragk_shifts<K>(lane, ksh);
+    // the fragment decode's two per-lane funnel shifts (the same for every tile and step) and its constants
+    uint32_t ksh[2];
+    frag_shifts<K>(lane, ksh);
+    const FragConsts fc = frag_consts();
     auto decode_a = [&](int slot, h8_t (&af)[4]) {
         const uint32_t* tw = reinterpret_cast<const uint32_t*>(lds + slot * STAGE + MATS * XBUF);
-        if constexpr (K == 4) {
 #pragma unroll
-            for (int t4 = 0; t4 < 4; ++t4) af[t4] = a_fragment4(tw + (stile0 + t4) * 64, lane);
-        } else {
-#pragma unroll
-            for (int t4 = 0; t4 < 4; ++t4) af[t4] = a_fragmentk<K>(tw + (stile0 + t4) * (16 * K), lane, ksh);
+        for (int t4 = 0; t4 < 4; ++t4) {
+            uint32_t wd[4];
+            frag_words<K>(tw + (stile0 + t4) * (16 * K), lane, wd);
+            af[t4] = a_fragment<K>(wd, ksh, fc);
         }
     };
 
@@ -764,19 +764,14 @@ __global__ void __launch_bounds__(256, BM == 256 ? 1 : 2) prefill_gemm_kernel(co
             // the next step's decode spread over this step's MFMA groups (sched_barrier keeps each group together,
             // so the VALU of the decode issues while the matrix core works)
             const uint32_t* twn = reinterpret_cast<const uint32_t*>(lds + sn * STAGE + MATS * XBUF);
-            uint32_t wp[4], w0[4], w1[4], st[4];
-            uint32_t wk[2][K == 4 ? 1 : 4];                // K = 3, 5: words of two tiles, one read ahead
+            uint32_t wd[K == 4 ? 4 : 2][4], W[2];          // K != 4: words of two tiles, one read ahead
             // the row-block count as an SGPR value opaque to the compiler at every step: each block's test is then
             // one s_cmp / s_cbranch_scc; left visible, the tests are hoisted out of the loop as lane masks and each
             // is rebuilt in the loop with a v_cndmask and a v_cmp (22 VALU instructions a step at 11 blocks)
             int nbs = nblk;
             __asm__ volatile("" : "+s"(nbs));
-            if constexpr (K == 4) {
 #pragma unroll
-                for (int t4 = 0; t4 < 4; ++t4) frag4_words(twn + (stile0 + t4) * 64, lane, wp[t4], w0[t4], w1[t4]);
-            } else {
-                fragk_words<K>(twn + stile0 * (16 * K), lane, wk[0]);
-            }
+            for (int t4 = 0; t4 < (K == 4 ? 4 : 1); ++t4) frag_words<K>(twn + (stile0 + t4) * (16 * K), lane, wd[t4]);
 #pragma unroll
             for (int b = 0; b < RB; ++b) {
                 const h8_t bc = ring[b % D];
@@ -790,14 +785,11 @@ __global__ void __launch_bounds__(256, BM == 256 ? 1 : 2) prefill_gemm_kernel(co
                 for (int pr = b * 16 / RB; pr < (b + 1) * 16 / RB; ++pr) {   // the 16 decoded pairs spread evenly
                     const int t = pr >> 2, j = pr & 3;
                     if (j == 0) {
-                        if constexpr (K == 4) {
-                            frag4_states(wp[t], w0[t], w1[t], lane, st);
-                        } else {
-                            fragk_states<K>(wk[t & 1], ksh, st);
-                            if (t < 3) fragk_words<K>(twn + (stile0 + t + 1) * (16 * K), lane, wk[(t + 1) & 1]);
-                        }
+                        frag_funnel<K>(wd[K == 4 ? t : t & 1], ksh, W);
+                        if (K != 4 && t < 3)
+                            frag_words<K>(twn + (stile0 + t + 1) * (16 * K), lane, wd[(t + 1) & 1]);
                     }
-                    const h2_t v = decode_pair(st[j]);
+                    const h2_t v = j & 1 ? frag_pair<K, 1>(W[j >> 1], fc) : frag_pair<K, 0>(W[j >> 1], fc);
                     an[t][2 * j] = v[0];
                     an[t][2 * j + 1] = v[1];
                 }
