@@ -50,6 +50,16 @@ namespace gfr {
 #endif
 constexpr int PF_BM2 = PF_BM2_ROWS, PF_BM3 = PF_BM3_ROWS, PF_BM4 = PF_BM4_ROWS, PF_BM5 = PF_BM5_ROWS;
 constexpr int pf_bm_for(int bits) { return bits == 2 ? PF_BM2 : bits == 3 ? PF_BM3 : bits == 4 ? PF_BM4 : PF_BM5; }
+// The item's rows pick one of the kernel's bodies: up to PF_SMALL rows, up to PF_MID, or the full item. A body of fewer
+// rows stages fewer bytes a step, so the same LDS keeps more steps in flight: the full 176-row body waits for loads it
+// issued one step before (three stages), the 32-row body for ones of six steps before, which an expert's first pass over
+// its trellis in HBM needs. Measured against one body (us a layer): 4096 rows of the FP8-shared geometry (median 34 rows
+// an expert) 1250 -> 1208; 1500 rows, hidden 5120, K = 3 1504 -> 1453.
+constexpr int PF_SMALL = 32, PF_MID = 96;
+// Windows of few rows an expert run PF_FEW-row items on kernels small enough for three workgroups a CU (168 VGPRs,
+// 53 KB of LDS): their programs are bound by the trellis decode's VALU work next to the stage waits, which a third wave a
+// SIMD covers. See window_form for where this form is taken and what it measured.
+constexpr int PF_FEW = 96, PF_FEW_OCC = 3;
 constexpr int PF_MAXU = 1024;       // distinct experts a window (grid / plan bound)
 
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -547,20 +557,17 @@ __device__ __forceinline__ h8_t a_fragment(const uint32_t (&wd)[4], const uint32
     return f;
 }
 
-// 16-byte direct-to-LDS load: lane i's 16 bytes land at lds_base + 16 i (lds_base uniform). Written as inline asm:
-// the compiler treats its builtin as an LDS store of unknown address and puts s_waitcnt vmcnt(0) before every later
-// LDS read, which drains the whole load pipeline each step; here the kernels wait for their stages themselves
-// (wait_vmcnt), and loads complete in order, so any wait the compiler adds for its own loads only waits longer.
-__device__ __forceinline__ void load_lds16(const void* g, void* lds_base) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(
-        (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds_base);
-    __asm__ volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "{m0}"(m0) : "memory");
-}
-
-// The same load in the scalar-base form: lane i reads sbase + voff_i (32-bit unsigned per-lane offset), so a
-// per-step advance is one 64-bit scalar add and the LDS destination (m0) stays in scalar registers.
-__device__ __forceinline__ void load_lds16_s(uint64_t sbase, uint32_t voff, uint32_t m0) {
-    __asm__ volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(voff), "s"(sbase), "{m0}"(m0) : "memory");
+// 16-byte direct-to-LDS load in the scalar-base form: lane i reads sbase + voff_i (32-bit unsigned per-lane offset) and
+// its 16 bytes land at m0 + 16 i, so a per-step advance is one 64-bit scalar add and the LDS destination stays in
+// scalar registers. Only the lanes of `mask` (uniform) load; the others' 16 bytes of LDS keep what they hold. An empty
+// mask still counts as one load (vmcnt), so every wave's count a step is the same whatever it has to load. Called with
+// all lanes active. Written as inline asm: the compiler treats its builtin as an LDS store of unknown address and puts
+// s_waitcnt vmcnt(0) before every later LDS read, which drains the whole load pipeline each step; here the kernels wait
+// for their stages themselves (wait_vmcnt), and loads complete in order, so any wait the compiler adds for its own loads
+// only waits longer.
+__device__ __forceinline__ void load_lds16_s(uint64_t sbase, uint32_t voff, uint32_t m0, uint64_t mask) {
+    __asm__ volatile("s_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1"
+                     :: "v"(voff), "s"(sbase), "{m0}"(m0), "s"(mask) : "memory");
 }
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
     // readfirstlane returns int: through uint32_t, so that the low word is not sign-extended into the high one
@@ -585,58 +592,45 @@ __device__ __forceinline__ void wait_vmcnt() {
 // columns (4 trellis tiles) x BM rows: a step of 32 k is 4 A fragments decoded in registers against BM / 16 B
 // fragments, so every decoded fragment feeds BM / 16 MFMAs. Software pipeline: while step s multiplies, the wave
 // decodes step s + 1's A fragments into a second register set and keeps a ring of B fragments D reads ahead of the
-// MFMAs; direct-to-LDS loads run NS - 1 steps ahead of the step that reads them. With BM = 128 two workgroups share
+// MFMAs; direct-to-LDS loads run NS - 1 steps ahead of the step that reads them. Two or three workgroups share
 // a CU, so one wave's decode (VALU) overlaps the other's MFMAs on each SIMD. A staged row keeps its four 16-byte
 // chunks XOR-swizzled by (row >> 1) & 3 to spread the B-fragment reads over the banks.
 // SPLIT: (item, column group, K split) programs over a.sk contiguous k ranges, each writing its raw partial sums to
 // a.z in the decode path's split layout (its epilogue kernels add the splits in order); for windows too small to
 // fill the GPU with full-K items.
-template <int MATS, int K, int BM, bool SPLIT = false>
-__global__ void __launch_bounds__(256, BM == 256 ? 1 : 2) prefill_gemm_kernel(const PrefillArgs a) {
-    constexpr int NCOLS = MATS == 2 ? 128 : 256, RB = BM / 16;
-    constexpr int OCC = BM == 256 ? 1 : 2;
-    constexpr int NS = SPLIT ? 4 : OCC == 1 ? (MATS == 2 ? 4 : 6) : (MATS == 2 ? 3 : 4);
-    constexpr int XBUF = BM * 64;                        // one matrix's rows of a step (2 k tiles, pair order)
-    constexpr int TBUF = 16 * 2 * 32 * K;                // the workgroup's 16 tiles x 2 k tiles of words
-    constexpr int STAGE = MATS * XBUF + TBUF;
-    constexpr int ER = BM % 64 ? 32 : BM / 4, EPITCH = 256 + 8;   // epilogue: ER rows of 256 fp32 columns at a time
-    constexpr int LDS_EPI = SPLIT ? 0 : ER * EPITCH * 4;
-    constexpr int LDS_BYTES = NS * STAGE > LDS_EPI ? NS * STAGE : LDS_EPI;
-    constexpr int XLOADS = (MATS * RB + 3) / 4;          // direct loads of rows a wave a step (the last repeated)
-    constexpr int TL = (K + 3) / 4;                      // direct loads of trellis words a wave a step
-    constexpr int LOADS = XLOADS + TL;
-    static_assert((BM == 256 || BM == 176 || BM == 160 || BM == 144 || BM == 128 || BM == 32) && NS <= 8, "tile shape");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
-    __shared__ int rows_sh[BM];
+// One program's place in the window: expert e, its member rows [.., + nrows) in rows_sh, column group, K split.
+struct GemmItem {
+    int e, nrows, cg, split;
+};
 
-    const int ncg = a.N / NCOLS;
-    // XCD-aware order: the hardware deals consecutive workgroups to the 8 XCDs in turn; renumber so that each XCD gets
-    // a contiguous range of (item, column group[, split]) -- an item's column groups then share one L2 (its token
-    // rows). The grid is sized for the most items a window can have; the window's real programs (nact, known once
-    // the plan has run) are spread over all 8 XCDs, taken by the first-dispatched workgroups.
+// Staged steps of a body: as many as a workgroup's share of the LDS holds (its rows_sh aside), at most 8, even from 4 on
+// (the unrolled main loop is a multiple of it).
+constexpr int gemm_stage_bytes(int mats, int K, int rows) { return mats * rows * 64 + 16 * 2 * 32 * K; }
+constexpr int gemm_stages(int mats, int K, int rows, int bm, int occ) {
+    const int n = (163840 / occ - bm * 4) / gemm_stage_bytes(mats, K, rows);
+    return n >= 8 ? 8 : n < 4 ? n : n & ~1;
+}
+constexpr int GEMM_EPITCH = 256 + 8, GEMM_ER = 32;       // epilogue: ER rows of 256 fp32 columns at a time
+
+// BM: rows the body stages and multiplies a step (the item's rows are at most this many).
+template <int MATS, int K, int BM, bool SPLIT, int NS>
+__device__ __forceinline__ void gemm_body(const PrefillArgs& a, unsigned char* lds, const int* rows_sh,
+                                          const GemmItem& item) {
+    constexpr int NCOLS = MATS == 2 ? 128 : 256, RB = BM / 16;
+    constexpr int XBUF = BM * 64;                        // one matrix's rows of a step (2 k tiles, pair order)
+    constexpr int STAGE = gemm_stage_bytes(MATS, K, BM);
+    constexpr int ER = GEMM_ER, EPITCH = GEMM_EPITCH;
+    constexpr int XLOADS = (MATS * RB + 3) / 4;          // direct loads of rows a wave a step
+    constexpr int TCH = 64 * K / MATS, TM = (TCH + 63) / 64;   // trellis words of a step: 16-byte chunks, loads a matrix
+    constexpr int TL = (MATS * TM + 3) / 4;              // direct loads of trellis words a wave a step
+    constexpr int LOADS = XLOADS + TL;
+    static_assert(BM % 16 == 0 && BM <= 176 && NS >= 3 && NS <= 8, "tile shape");
     const int nsk = SPLIT ? a.sk : 1;
-    const int nact = a.plan[0] * ncg * nsk, per = (nact + 7) >> 3;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int full = nact & 7 ? nact & 7 : 8;            // XCDs holding `per` programs (the rest hold per - 1)
-    if (slot >= (xcd < full ? per : per - 1)) return;
-    const int logical = (xcd < full ? xcd * per : full * per + (xcd - full) * (per - 1)) + slot;
-    const int item = logical / (ncg * nsk), cg = logical / nsk % ncg, split = logical % nsk;
-    const int it = a.items[item];
-    const int u = it >> 16, pass = it & 0xffff;
-    const int e = a.uids[u];
-    // the expert's members split evenly over its ceil(cnt / BM) passes; row blocks past nrows skip their MFMAs
-    const int ucnt = a.ucnt[u], npass = (ucnt + BM - 1) / BM;
-    const int rbeg = pass * ucnt / npass, nrows = (pass + 1) * ucnt / npass - rbeg;
-    const int nblk = (nrows + 15) >> 4;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    {
-        const int* mrow = a.members + (size_t)u * a.maxm + rbeg;
-        const int c0 = mrow[0];
-        const int p0 = (c0 >> 5) * a.slots + (c0 & 31);
-        const int code = tid < nrows ? mrow[tid] : -1;
-        if (tid < BM) rows_sh[tid] = code >= 0 ? (code >> 5) * a.slots + (code & 31) : p0;   // padding: member 0
-    }
-    __syncthreads();
+    const int e = item.e, nrows = item.nrows, cg = item.cg, split = item.split;
+    const int nblk = (nrows + 15) >> 4;                  // row blocks past nrows skip their MFMAs
+    int tid = threadIdx.x;
+    __asm__ volatile("" : "+v"(tid));                    // a body's lane values stay its own: shared by the bodies of a
+    const int wave = tid >> 6, lane = tid & 63;          // kernel they are held across all of them and spill
 
     const int KT = a.Kin >> 4, NT = a.N >> 4, S = KT / 2 / nsk, s0 = split * S;   // this program's steps s0 ..
     const int col0 = cg * NCOLS;
@@ -649,7 +643,7 @@ __global__ void __launch_bounds__(256, BM == 256 ? 1 : 2) prefill_gemm_kernel(co
     // 2^32); the LDS destinations are uniform too
     const int wv = __builtin_amdgcn_readfirstlane(wave);
     const uint32_t lds_u = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds;
-    uint64_t xbase[XLOADS];
+    uint64_t xbase[XLOADS], xmask[XLOADS];
     uint32_t xoff[XLOADS];
 #pragma unroll
     for (int j = 0; j < XLOADS; ++j) {
@@ -658,44 +652,34 @@ __global__ void __launch_bounds__(256, BM == 256 ? 1 : 2) prefill_gemm_kernel(co
         const int c = pos ^ ((row >> 1) & 3);              // the global chunk this LDS position holds
         xbase[j] = uniform64((uint64_t)(uintptr_t)(m ? a.x1 : a.x0) + (uint64_t)s0 * 64);
         xoff[j] = (uint32_t)rows_sh[row] * (uint32_t)(a.Kin * 2) + (uint32_t)((c >> 1) * 32 + (c & 1) * 16);
+        // rows past the item's, and block numbers past the stage's, load nothing (a row's products only enter its own
+        // outputs, and a row past nrows is never stored)
+        xmask[j] = uniform64(wv * XLOADS + j < MATS * RB ? __ballot(row < nrows) : 0);
     }
-    // trellis words: 32 blocks (tile, k tile) of 32 K bytes, K loads of 64 16-byte chunks; wave w issues loads
-    // w, w + 4, ... (the last one repeated where K is not a multiple of 4: the same bytes to the same place). The
-    // matrix of a load is uniform unless a load straddles the gate / up halves (MATS = 2, K = 3 or 5): then the
-    // lanes keep 64-bit addresses.
-    constexpr bool TUNI = MATS == 1 || K == 2 || K == 4;
-    const uint32_t* tsrc[TL];
-    uint64_t tbase[TL];
-    uint32_t toff[TL];
-    int tdst[TL];
+    // trellis words: 32 / MATS blocks (tile, k tile) of 32 K bytes a matrix, TM loads of 64 16-byte chunks each (the last
+    // one's lanes past the matrix's chunks load nothing, so that a load's matrix is uniform); wave w issues loads
+    // w, w + 4, ..., past the last one empty, so that every wave counts TL
+    uint64_t tbase[TL], tmask[TL];
+    uint32_t toff[TL], tdst[TL];
 #pragma unroll
     for (int j = 0; j < TL; ++j) {
-        const int li = wv + 4 * j < K ? wv + 4 * j : K - 1;
-        const int c = li * 64 + lane, blk = c / (2 * K), ch = c % (2 * K);
-        const int tile = blk >> 1, kt = blk & 1;
-        const int tmat = MATS == 2 ? tile >> 3 : 0;
-        const int ntile = col0 / 16 + (MATS == 2 ? (tile & 7) : tile);
-        const uint32_t* tm = tmat ? a.t1 : a.t0;
-        if constexpr (TUNI) {
-            tbase[j] = uniform64((uint64_t)(uintptr_t)tm + (uint64_t)s0 * 2 * NT * (8 * K) * 4);
-            toff[j] = (uint32_t)((((e * KT + kt) * NT + ntile) * (8 * K) + ch * 4) * 4);
-        } else {
-            tsrc[j] = tm + (((size_t)e * KT + 2 * s0 + kt) * NT + ntile) * (8 * K) + ch * 4;
-        }
-        tdst[j] = MATS * XBUF + li * 1024;
+        const int li = wv + 4 * j < MATS * TM ? wv + 4 * j : 0, tmat = li / TM;
+        const int c = li % TM * 64 + lane, blk = c / (2 * K), ch = c % (2 * K);
+        const int ntile = col0 / 16 + (blk >> 1), kt = blk & 1;
+        tmask[j] = uniform64(wv + 4 * j < MATS * TM ? __ballot(c < TCH) : 0);
+        tbase[j] = uniform64((uint64_t)(uintptr_t)(tmat ? a.t1 : a.t0) + (uint64_t)s0 * 2 * NT * (8 * K) * 4);
+        toff[j] = (uint32_t)((((e * KT + kt) * NT + ntile) * (8 * K) + ch * 4) * 4);
+        tdst[j] = MATS * XBUF + (tmat * TCH + li % TM * 64) * 16;
     }
     auto issue = [&](int s) {
         const uint32_t st = lds_u + (uint32_t)((s % NS) * STAGE);
 #pragma unroll
         for (int j = 0; j < XLOADS; ++j)
-            load_lds16_s(xbase[j] + (uint64_t)s * 64, xoff[j], st + min(wv * XLOADS + j, MATS * RB - 1) * 1024);
+            load_lds16_s(xbase[j] + (uint64_t)s * 64, xoff[j], st + min(wv * XLOADS + j, MATS * RB - 1) * 1024,
+                         xmask[j]);
 #pragma unroll
-        for (int j = 0; j < TL; ++j) {
-            if constexpr (TUNI)
-                load_lds16_s(tbase[j] + (uint64_t)s * 2 * NT * (8 * K) * 4, toff[j], st + tdst[j]);
-            else
-                load_lds16(tsrc[j] + (size_t)s * 2 * NT * (8 * K), lds + (s % NS) * STAGE + tdst[j]);
-        }
+        for (int j = 0; j < TL; ++j)
+            load_lds16_s(tbase[j] + (uint64_t)s * 2 * NT * (8 * K) * 4, toff[j], st + tdst[j], tmask[j]);
     };
     // wait until at most n stages' loads of this wave are outstanding
     static_assert(NS - 2 <= 6 && 6 * LOADS < 64, "vmcnt range");
@@ -958,6 +942,58 @@ __global__ void __launch_bounds__(256, BM == 256 ? 1 : 2) prefill_gemm_kernel(co
     chunk(std::integral_constant<int, 5>{});
 }
 
+// OCC: workgroups a CU. Full-K forms: the item's rows pick the body.
+template <int MATS, int K, int BM, bool SPLIT, int OCC>
+__global__ void __launch_bounds__(256, OCC) prefill_gemm_kernel(const PrefillArgs a) {
+    constexpr int NCOLS = MATS == 2 ? 128 : 256;
+    constexpr bool BODIES = !SPLIT, MID = BODIES && OCC == 2;
+    static_assert(SPLIT || (PF_SMALL < BM && (OCC != 2 || PF_MID < BM)), "a body reads rows_sh up to its own rows");
+    constexpr int NSB = SPLIT ? 4 : gemm_stages(MATS, K, BM, BM, OCC);
+    constexpr int NSM = gemm_stages(MATS, K, PF_MID, BM, OCC), NSS = gemm_stages(MATS, K, PF_SMALL, BM, OCC);
+    constexpr int cmax[4] = {NSB * gemm_stage_bytes(MATS, K, BM), MID ? NSM * gemm_stage_bytes(MATS, K, PF_MID) : 0,
+                             BODIES ? NSS * gemm_stage_bytes(MATS, K, PF_SMALL) : 0,
+                             SPLIT ? 0 : GEMM_ER * GEMM_EPITCH * 4};
+    constexpr int m0 = cmax[0] > cmax[1] ? cmax[0] : cmax[1], m1 = cmax[2] > cmax[3] ? cmax[2] : cmax[3];
+    constexpr int LDS_BYTES = m0 > m1 ? m0 : m1;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
+    __shared__ int rows_sh[BM];
+
+    const int ncg = a.N / NCOLS;
+    // XCD-aware order: the hardware deals consecutive workgroups to the 8 XCDs in turn; renumber so that each XCD gets
+    // a contiguous range of (item, column group[, split]) -- an item's column groups then share one L2 (its token
+    // rows). The grid is sized for the most items a window can have; the window's real programs (nact, known once
+    // the plan has run) are spread over all 8 XCDs, taken by the first-dispatched workgroups.
+    const int nsk = SPLIT ? a.sk : 1;
+    const int nact = a.plan[0] * ncg * nsk, per = (nact + 7) >> 3;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int full = nact & 7 ? nact & 7 : 8;            // XCDs holding `per` programs (the rest hold per - 1)
+    if (slot >= (xcd < full ? per : per - 1)) return;
+    const int logical = (xcd < full ? xcd * per : full * per + (xcd - full) * (per - 1)) + slot;
+    const int it = a.items[logical / (ncg * nsk)];
+    const int u = it >> 16, pass = it & 0xffff;
+    // the expert's members split evenly over its ceil(cnt / BM) passes
+    const int ucnt = a.ucnt[u], npass = (ucnt + BM - 1) / BM;
+    const int rbeg = pass * ucnt / npass, nrows = (pass + 1) * ucnt / npass - rbeg;
+    const GemmItem item{__builtin_amdgcn_readfirstlane(a.uids[u]), __builtin_amdgcn_readfirstlane(nrows),
+                        logical / nsk % ncg, logical % nsk};
+    {
+        const int tid = threadIdx.x;
+        const int* mrow = a.members + (size_t)u * a.maxm + rbeg;
+        const int c0 = mrow[0];
+        const int p0 = (c0 >> 5) * a.slots + (c0 & 31);
+        const int code = tid < nrows ? mrow[tid] : -1;
+        if (tid < BM) rows_sh[tid] = code >= 0 ? (code >> 5) * a.slots + (code & 31) : p0;   // padding: member 0
+    }
+    __syncthreads();
+    if constexpr (BODIES) {
+        if (item.nrows <= PF_SMALL) return gemm_body<MATS, K, PF_SMALL, false, NSS>(a, lds, rows_sh, item);
+    }
+    if constexpr (MID) {
+        if (item.nrows <= PF_MID) return gemm_body<MATS, K, PF_MID, false, NSM>(a, lds, rows_sh, item);
+    }
+    gemm_body<MATS, K, BM, SPLIT, NSB>(a, lds, rows_sh, item);
+}
+
 }  // namespace gfr
 
 struct gfr_fast_experts {
@@ -984,7 +1020,7 @@ constexpr int PF_SPLIT_K = 512;
 static int split_k_gateup(int hidden) { return hidden % (2 * PF_SPLIT_K) == 0 ? 2 * PF_SPLIT_K : PF_SPLIT_K; }
 constexpr int PF_SPLIT_BM = 32;
 static bool split_ok(int hidden, int inter) { return hidden % PF_SPLIT_K == 0 && inter % PF_SPLIT_K == 0; }
-static_assert(PF_SPLIT_BM <= PF_BM2 && PF_SPLIT_BM <= PF_BM3 && PF_SPLIT_BM <= PF_BM4 && PF_SPLIT_BM <= PF_BM5,
+static_assert(PF_SPLIT_BM <= PF_FEW && PF_SPLIT_BM <= PF_BM2 && PF_SPLIT_BM <= PF_BM3 && PF_SPLIT_BM <= PF_BM4 && PF_SPLIT_BM <= PF_BM5,
               "items are bounded at the smallest item size");
 // The most items a window of P pairs over at most maxu distinct experts can plan, at any item size the engine uses.
 static size_t item_bound(size_t P, size_t maxu) {
@@ -1024,25 +1060,44 @@ hipError_t prefill_create(gfr_fast_experts** out, int hidden, int inter, int slo
 
 PrefillDims prefill_dims(const gfr_fast_experts* fx) { return fx->d; }
 
-template <int MATS>
-static hipError_t launch_gemm_split(int bits, dim3 grid, hipStream_t s, const PrefillArgs& a) {
-    switch (bits) {
-        case 2: prefill_gemm_kernel<MATS, 2, PF_SPLIT_BM, true><<<grid, 256, 0, s>>>(a); break;
-        case 3: prefill_gemm_kernel<MATS, 3, PF_SPLIT_BM, true><<<grid, 256, 0, s>>>(a); break;
-        case 4: prefill_gemm_kernel<MATS, 4, PF_SPLIT_BM, true><<<grid, 256, 0, s>>>(a); break;
-        case 5: prefill_gemm_kernel<MATS, 5, PF_SPLIT_BM, true><<<grid, 256, 0, s>>>(a); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+// The window's form, from its pairs P and the engine's experts E (the same rule for the plan and the launches):
+//   SPLIT  split-K programs: windows whose full-K programs would leave CUs idle behind a few long ones;
+//   FEW    full-K items of up to PF_FEW rows, three workgroups a CU;
+//   LARGE  full-K items of pf_bm_for rows, two a CU: each decoded weight feeds more rows.
+// Up to PF_SPLIT_PAIRS pairs, FEW needs some rows an expert and gate/up programs for two rounds of 768 (us a layer,
+// split / few): hidden 5120, 160 + 1 experts, top-8: 64 rows 462 / 485, 77 rows (K = 3) 513 / 528, 100 rows 579 / 580
+// (K = 3) and 658 / 647 (uniform), 150 rows 711 / 656, 220 rows (K = 2) 773 / 685; fewer programs: hidden 2048, 64 + 1,
+// top-4, 300 rows 179 / 197 (uniform) and 200 / 193, hidden 4096, 288 experts, top-8, inter 512, 220 rows (K = 2) 412 /
+// 415. From PF_FEW_MEAN rows an expert LARGE wins where an expert's rows fit one of its passes (us a layer, few /
+// large): 16 (512 rows, 288 experts) 429 / 502; 77 (1000 rows, hidden 2048) 248 / 323; 84 (1500 rows, hidden 5120,
+// K = 3) 1405 / 1491; 94 (3000 rows, 288 experts) 979 / 1031; 112 (2000 rows, hidden 5120, uniform) 1798 / 1589; 630
+// (8192 rows, hidden 2048) 1323 / 1181.
+constexpr int PF_FEW_MEAN = 100;
+enum class Form { SPLIT, FEW, LARGE };
+static Form window_form(const gfr_fast_experts* fx, int rows) {
+    const int P = rows * fx->d.slots, E = fx->d.experts;
+    const int programs = (fx->d.inter / 128) * ((P < E ? P : E) + P / PF_FEW);
+    const bool many = P >= 6 * E && programs >= 2 * 3 * 256;
+    if (fx->zgu && P <= PF_SPLIT_PAIRS && !many) return Form::SPLIT;
+    return P < PF_FEW_MEAN * E ? Form::FEW : Form::LARGE;
+}
+static int form_rows(Form f, int bits) {
+    return f == Form::SPLIT ? PF_SPLIT_BM : f == Form::FEW ? PF_FEW : pf_bm_for(bits);
 }
 
+template <int MATS, int K, int BM>
+static void launch_gemm_k(Form f, dim3 grid, hipStream_t s, const PrefillArgs& a) {
+    if (f == Form::SPLIT) prefill_gemm_kernel<MATS, K, PF_SPLIT_BM, true, 2><<<grid, 256, 0, s>>>(a);
+    else if (f == Form::FEW) prefill_gemm_kernel<MATS, K, PF_FEW, false, PF_FEW_OCC><<<grid, 256, 0, s>>>(a);
+    else prefill_gemm_kernel<MATS, K, BM, false, 2><<<grid, 256, 0, s>>>(a);
+}
 template <int MATS>
-static hipError_t launch_gemm(int bits, dim3 grid, hipStream_t s, const PrefillArgs& a) {
+static hipError_t launch_gemm(Form f, int bits, dim3 grid, hipStream_t s, const PrefillArgs& a) {
     switch (bits) {
-        case 2: prefill_gemm_kernel<MATS, 2, PF_BM2><<<grid, 256, 0, s>>>(a); break;
-        case 3: prefill_gemm_kernel<MATS, 3, PF_BM3><<<grid, 256, 0, s>>>(a); break;
-        case 4: prefill_gemm_kernel<MATS, 4, PF_BM4><<<grid, 256, 0, s>>>(a); break;
-        case 5: prefill_gemm_kernel<MATS, 5, PF_BM5><<<grid, 256, 0, s>>>(a); break;
+        case 2: launch_gemm_k<MATS, 2, PF_BM2>(f, grid, s, a); break;
+        case 3: launch_gemm_k<MATS, 3, PF_BM3>(f, grid, s, a); break;
+        case 4: launch_gemm_k<MATS, 4, PF_BM4>(f, grid, s, a); break;
+        case 5: launch_gemm_k<MATS, 5, PF_BM5>(f, grid, s, a); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1094,8 +1149,8 @@ hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_exper
                                                                    d.exl3_slots, mats);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    const bool split = fx->zgu && P <= PF_SPLIT_PAIRS;
-    const int bm = split ? PF_SPLIT_BM : pf_bm_for(w->bits);
+    const Form form = window_form(fx, rows);
+    const int bm = form_rows(form, w->bits);
     if (!planned) {
         prefill_plan_kernel<<<1, 1024, 0, s>>>(ids, count, members, maxm, w->experts, maxu, bm, fx->ucnt, fx->items,
                                                fx->plan);
@@ -1107,18 +1162,18 @@ hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_exper
     PrefillArgs a{};
     a.uids = ids; a.members = members; a.ucnt = fx->ucnt; a.items = fx->items; a.plan = fx->plan;
     a.maxm = maxm; a.slots = d.slots; a.limit = 10.f;
-    if (split) {
+    if (form == Form::SPLIT) {
         // gate / up partials -> epilogue (xd in pair order) -> down partials -> epilogue -> output
         const int skg = d.hidden / split_k_gateup(d.hidden), skd = d.inter / PF_SPLIT_K;
         a.sk = skg; a.P = P; a.z = fx->zgu;
         a.x0 = fx->xg; a.x1 = shared_x ? fx->xg : fx->xu; a.t0 = w->gt; a.t1 = w->ut; a.Kin = d.hidden; a.N = d.inter;
-        if ((e = launch_gemm_split<2>(w->bits, dim3(max_items * (d.inter / 128) * skg), s, a)) != hipSuccess) return e;
+        if ((e = launch_gemm<2>(form, w->bits, dim3(max_items * (d.inter / 128) * skg), s, a)) != hipSuccess) return e;
         if ((e = launch_gateup_epilogue(s, fx->zgu, picks, w->svh_g, w->svh_u, w->suh_d, fx->xd, P, d.inter, skg,
                                         d.slots, d.exl3_slots, 10.f, true)) != hipSuccess)
             return e;
         a.sk = skd; a.z = fx->zd;
         a.x0 = fx->xd; a.x1 = fx->xd; a.t0 = w->dt; a.t1 = w->dt; a.Kin = d.inter; a.N = d.hidden;
-        if ((e = launch_gemm_split<1>(w->bits, dim3(max_items * (d.hidden / 256) * skd), s, a)) != hipSuccess) return e;
+        if ((e = launch_gemm<1>(form, w->bits, dim3(max_items * (d.hidden / 256) * skd), s, a)) != hipSuccess) return e;
         if (combine_weights && combine_out && d.exl3_slots <= 16) {
             // the down epilogue and the layer's slot-ordered combine in one launch (the decode path's finish)
             if (combined) *combined = true;
@@ -1131,17 +1186,16 @@ hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_exper
     // gate / up -> xd
     a.x0 = fx->xg; a.x1 = shared_x ? fx->xg : fx->xu; a.t0 = w->gt; a.t1 = w->ut; a.Kin = d.hidden; a.N = d.inter;
     a.sv0 = w->svh_g; a.sv1 = w->svh_u; a.sd = w->suh_d; a.xd = fx->xd; a.y = fx->out;
-    if ((e = launch_gemm<2>(w->bits, dim3(max_items * (d.inter / 128)), s, a)) != hipSuccess) return e;
+    if ((e = launch_gemm<2>(form, w->bits, dim3(max_items * (d.inter / 128)), s, a)) != hipSuccess) return e;
     // down -> output
     a.x0 = fx->xd; a.x1 = fx->xd; a.t0 = w->dt; a.t1 = w->dt; a.Kin = d.inter; a.N = d.hidden;
     a.sv0 = w->svh_d; a.sv1 = nullptr; a.sd = nullptr; a.xd = nullptr; a.y = fx->out;
-    return launch_gemm<1>(w->bits, dim3(max_items * (d.hidden / 256)), s, a);
+    return launch_gemm<1>(form, w->bits, dim3(max_items * (d.hidden / 256)), s, a);
 }
 
 float* prefill_output(const gfr_fast_experts* fx) { return fx->out; }
 int prefill_item_rows(const gfr_fast_experts* fx, int rows, int bits) {
-    const bool split = fx->zgu && rows * fx->d.slots <= PF_SPLIT_PAIRS;
-    return split ? PF_SPLIT_BM : pf_bm_for(bits);
+    return form_rows(window_form(fx, rows), bits);
 }
 hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_experts* w,
                                   const uint16_t* input, int input_stride, const float* logits, int rows, int routed,

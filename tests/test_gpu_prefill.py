@@ -315,3 +315,34 @@ def test_split_window_with_many_experts(gfr, oracle):
         assert_close(out[r], want[0], what=f"token {r}")
     y = window_reference(oracle, w, x, p, workers=16)
     assert_rows_close(out, oracle.combine(y, wt, rows, topk + 1), what="1023 experts, every token")
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 5])
+@pytest.mark.parametrize("form,hidden,inter", [("few", 256, 256), ("few", 768, 512), ("large", 256, 256),
+                                               ("large", 1280, 256)])
+def test_prefill_item_bodies(gfr, oracle, bits, form, hidden, inter):
+    """Experts with member counts around every body's and item's rows (16-row blocks, the 32- and 96-row bodies, the
+    form's item), at K depths shorter and longer than the staged steps: every output against the oracle. Hidden sizes
+    that are not multiples of 512 have no split-K form; fewer than 100 pairs an expert run the few-row form."""
+    import synth
+    bm = {2: 176, 3: 160, 4: 176, 5: 144}[bits]
+    counts = [1, 15, 16, 17, 31, 32, 33, 95, 96, 97, 193] if form == "few" else [1, 32, 33, 96, 97, bm - 1, bm, bm + 1,
+                                                                              2 * bm + 1]
+    E, rows = len(counts), sum(counts)
+    assert (rows < 100 * E) == (form == "few")
+    rng = np.random.default_rng(bits)
+    picks_np = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(rows, 1)
+    picks = torch.from_numpy(picks_np).cuda()
+    w = synth.experts(E, hidden, inter, bits, seed=600 + bits)
+    x = synth.activations(rows, hidden, 31 + bits)
+    g = gfr.Grouping(E, 1, rows)
+    g.run(picks, rows)
+    fx = gfr.FastExperts(hidden, inter, 1, 1, E, rows)
+    fx.run(w, x, picks, g.ids, g.count, g.members, rows, rows, shared_x=False)
+    torch.cuda.synchronize()
+    # the sums' order differs from the oracle's, so an activation's bf16 rounding may go the other way: 2^-8 of one value
+    # of at most 150 (10 * 10 * a suh_d of 1.5) in a row whose norm is about 80 sqrt(inter / 2) (half the gates are
+    # negative); nine of them add up to three
+    bound = 3 * 2.0 ** -8 * 150 / (80 * (inter / 2) ** 0.5)
+    assert_rows_close(fx.output[:rows].cpu().numpy(), window_reference(oracle, w, x, picks_np).reshape(rows, hidden),
+                      rel_rms=bound, what=f"{form} K={bits} {hidden}x{inter}")
