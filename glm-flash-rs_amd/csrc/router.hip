@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "route.hpp"
 
 namespace gfr {
@@ -121,6 +123,103 @@ __global__ void __launch_bounds__(256) router_logits_kernel(const uint16_t* __re
     }
 }
 
+// The same product on the matrix core, for windows of many rows: v_mfma_f32_16x16x32_bf16 with 16 experts as A and 16
+// rows as B, fragments loaded straight from memory (a 64-k chunk a round: lane (row or expert l % 16, q = l / 16) holds
+// k = 16 q .. 16 q + 15, 32 bytes; both operands take the chunk's k in that order, so each row's 128 bytes are one full
+// line). A workgroup owns RB x EB tiles over the whole K: its 8 waves take contiguous eighths of the chunks, in chains
+// of four MFMAs added in fp32, and the waves' sums meet in LDS in wave order in fp64 (error against fp64 7.7e-8 at
+// hidden 4096, 8.3e-8 for the lanes' dot products; chains of 16 with an fp32 sum 1.4e-7). Bound by the operand reads from
+// L2 (a row is read by E / (16 EB) workgroups, an expert by rows / (16 RB)), so the tiles are as large as the registers
+// allow (RB x EB = 4 x 5: two sums of 80 and 72 of loads) and one round of workgroups covers the window. Measured against
+// router_logits_kernel (us): 4096 rows, hidden 4096, 288 experts 202 -> 38; 8192 rows, hidden 5120, 160 experts 599 ->
+// 48; 700 rows 60 -> 15; 128 rows, 288 experts 12.9 -> 12.7; below that the dot products win (64 rows 9.6 against 12.6).
+constexpr int ROUTER_MFMA_ROWS = 128;
+typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+constexpr int ROUTER_WAVES = 8;
+template <int RB, int EB>
+__global__ void __launch_bounds__(64 * ROUTER_WAVES) router_mfma_kernel(const uint16_t* __restrict__ x, int x_stride,
+                                                                        const uint16_t* __restrict__ W, int D, int E,
+                                                                        int rows, float* __restrict__ logits) {
+    constexpr int GT = RB * EB < 8 ? RB * EB : 8;          // tiles of a reduction round
+    __shared__ f4_t part[ROUTER_WAVES][GT][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, a = lane & 15, q = lane >> 4;
+    const int e0 = blockIdx.x * 16 * EB, r0 = blockIdx.y * 16 * RB;
+    const int nc = (D + 63) / 64, c0 = wave * nc / ROUTER_WAVES, c1 = (wave + 1) * nc / ROUTER_WAVES;
+    // rows and experts past the end repeat the last one (their results are not stored)
+    const uint16_t *wp[EB], *xp[RB];
+#pragma unroll
+    for (int i = 0; i < EB; ++i) wp[i] = W + (size_t)min(e0 + 16 * i + a, E - 1) * D + 16 * q;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) xp[i] = x + (size_t)min(r0 + 16 * i + a, rows - 1) * x_stride + 16 * q;
+    f4_t sum[EB][RB];
+#pragma unroll
+    for (int i = 0; i < EB; ++i)
+#pragma unroll
+        for (int j = 0; j < RB; ++j) sum[i][j] = (f4_t){0.f, 0.f, 0.f, 0.f};
+    for (int c = c0; c < c1; c += 2) {
+        f4_t acc[EB][RB];
+#pragma unroll
+        for (int i = 0; i < EB; ++i)
+#pragma unroll
+            for (int j = 0; j < RB; ++j) acc[i][j] = (f4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = (c + u) * 64;
+            auto load = [&](const uint16_t* p, bf8_t (&v)[2]) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    uint4 t = make_uint4(0u, 0u, 0u, 0u);
+                    if (c + u < c1 && k + 16 * q + 8 * h < D) t = *reinterpret_cast<const uint4*>(p + k + 8 * h);
+                    v[h] = __builtin_bit_cast(bf8_t, t);
+                }
+            };
+            bf8_t wv[EB][2], xv[RB][2];
+#pragma unroll
+            for (int i = 0; i < EB; ++i) load(wp[i], wv[i]);
+#pragma unroll
+            for (int j = 0; j < RB; ++j) load(xp[j], xv[j]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < RB; ++j)
+#pragma unroll
+                    for (int i = 0; i < EB; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i][h], xv[j][h], acc[i][j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < EB; ++i)
+#pragma unroll
+            for (int j = 0; j < RB; ++j) sum[i][j] += acc[i][j];
+    }
+    // D holds experts 4 q .. 4 q + 3 of the tile for row a: the waves' sums in order, GT tiles a round
+#pragma unroll
+    for (int g = 0; g < RB * EB; g += GT) {
+        if (g) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < GT; ++t)
+            if (g + t < RB * EB) part[wave][t][lane] = sum[(g + t) / RB][(g + t) % RB];
+        __syncthreads();
+        if (wave < GT && g + wave < RB * EB) {
+            double d[4] = {0., 0., 0., 0.};
+#pragma unroll
+            for (int w = 0; w < ROUTER_WAVES; ++w) {
+                const f4_t p = part[w][wave][lane];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) d[j] += (double)p[j];
+            }
+            const f4_t v = {(float)d[0], (float)d[1], (float)d[2], (float)d[3]};
+            const int e = e0 + (g + wave) / RB * 16 + 4 * q, r = r0 + (g + wave) % RB * 16 + a;
+            if (r < rows) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (e + j < E) logits[(size_t)r * E + e + j] = v[j];
+            }
+        }
+    }
+}
+
 }  // namespace gfr
 
 #include "launch.hpp"
@@ -144,6 +243,31 @@ int router_logits_max_hidden() { return 1 << 16; }
 
 hipError_t launch_router_logits(hipStream_t s, const uint16_t* x, int x_stride, const uint16_t* W, int D, int E,
                                 int rows, float* logits) {
+    if (rows >= ROUTER_MFMA_ROWS) {
+        // the tile with the lowest estimate: rounds of one workgroup a CU, each as long as its operand reads (rows and
+        // experts of a tile) plus a fixed part
+        const auto wgs = [&](int rb, int eb) { return (rows + 16 * rb - 1) / (16 * rb) * ((E + 16 * eb - 1) / (16 * eb)); };
+        const int tiles[5][2] = {{4, 5}, {4, 4}, {2, 4}, {2, 2}, {1, 2}};
+        int best = 0, cost = 0;
+        for (int t = 0; t < 5; ++t) {
+            const int c = (wgs(tiles[t][0], tiles[t][1]) + 255) / 256 * (tiles[t][0] + tiles[t][1] + 4);
+            if (t == 0 || c < cost) best = t, cost = c;
+        }
+        const auto go = [&](auto rb, auto eb) {
+            constexpr int RB = decltype(rb)::value, EB = decltype(eb)::value;
+            router_mfma_kernel<RB, EB><<<dim3((E + 16 * EB - 1) / (16 * EB), (rows + 16 * RB - 1) / (16 * RB)),
+                                         64 * ROUTER_WAVES, 0, s>>>(x, x_stride, W, D, E, rows, logits);
+            return hipGetLastError();
+        };
+        using std::integral_constant;
+        switch (best) {
+            case 0: return go(integral_constant<int, 4>{}, integral_constant<int, 5>{});
+            case 1: return go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+            case 2: return go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+            case 3: return go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+            default: return go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+        }
+    }
     const int RT = rows >= 64 ? ROUTER_RTMAX : rows >= 8 ? 4 : 1;
     router_logits_kernel<<<dim3((E + 7) / 8, (rows + RT - 1) / RT), 256, 0, s>>>(x, x_stride, W, D, E, rows, RT,
                                                                                   logits);

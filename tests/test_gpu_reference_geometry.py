@@ -99,6 +99,23 @@ def test_router_logits_vs_float64(gfr, rows, routed, hidden):
     assert np.all(err <= 1e-6 * scale + 1e-7), float((err / (scale + 1e-30)).max())
 
 
+@pytest.mark.parametrize("rows,routed,hidden", [(127, 33, 1032), (128, 33, 1032), (129, 1, 8), (257, 65, 72), (300, 64, 2048),
+                                                (1000, 81, 4104), (1025, 289, 136), (4097, 288, 520)])
+def test_router_logits_matrix_tiles(gfr, rows, routed, hidden):
+    """Row counts on both sides of the matrix-core form, and its tiles' edges: rows, experts and hidden sizes that end
+    inside a tile, a chunk or a wave's share, every logit against the float64 product. A 32-bit sum in any order is
+    within (hidden / 256 + 12) roundings (chains of four MFMAs a wave, the sums, the result) of 2^-24 of the sum of the
+    products' magnitudes."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn((rows, hidden), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((routed, hidden), generator=g, device="cuda").to(torch.bfloat16)
+    got = gfr.router_logits(x, w).double()
+    want = x.double() @ w.double().t()
+    mag = x.double().abs() @ w.double().abs().t()
+    assert ((got - want).abs() <= (hidden / 256 + 12) * 2.0 ** -24 * mag).all()
+
+
+
 @pytest.mark.parametrize("rows", [1, 3, 40, 300])
 def test_moe_reference_layout_shared_output(gfr, oracle, weights, rows):
     """Moe::run_prefetched at the reference's layout (moe.rs:77-181): router logits from the hidden rows, GLM's gate
