@@ -399,6 +399,38 @@ __global__ void __launch_bounds__(512) route_group_rot_kernel(const float* __res
                     suh0, suh1, out0, out1, K, row, bp, topk + 1, exl3_slots);
 }
 
+// group_small_kernel's work (with the item plan) in workgroup 0 and the rotation's tasks in the others, for windows
+// whose picks are routed: launch_route_group_rot's second launch where one workgroup's routing of every row would
+// outlast the rest.
+template <int MATS>
+__global__ void __launch_bounds__(512) group_small_rot_kernel(const int* __restrict__ picks, int rows, int slots, int E,
+                                                              int* __restrict__ ids, int* __restrict__ count,
+                                                              int* __restrict__ members, int maxm, int bm,
+                                                              int* __restrict__ plan_ucnt,
+                                                              int* __restrict__ plan_items, int* __restrict__ plan,
+                                                              int plan_E, const uint16_t* __restrict__ x, int x_stride,
+                                                              const uint16_t* __restrict__ suh0,
+                                                              const uint16_t* __restrict__ suh1,
+                                                              uint16_t* __restrict__ out0, uint16_t* __restrict__ out1,
+                                                              int K, int exl3_slots) {
+    extern __shared__ uint32_t lds[];
+    __shared__ __attribute__((aligned(16))) int scan_scratch[16];
+    if (blockIdx.x == 0) {
+        int* pk = reinterpret_cast<int*>(lds);               // [rows][slots], read many times below
+        for (int i = threadIdx.x; i < rows * slots; i += blockDim.x) pk[i] = picks[i];
+        __syncthreads();
+        group_small_body(pk, rows, slots, E, ids, count, members, maxm, lds + rows * slots, scan_scratch, bm, plan_ucnt,
+                         plan_items, plan, plan_E);
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    const int task = (blockIdx.x - 1) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int KP = K / 256, row = task / KP, bp = task % KP;
+    if (row >= rows) return;
+    rot2_task<MATS>(x, x_stride, [&] { return lane < exl3_slots ? picks[row * slots + lane] : 0; }, suh0, suh1, out0,
+                    out1, K, row, bp, slots, exl3_slots);
+}
+
 // The large-window grouping's scatter launch (group_scatter_body, workgroups 0 .. E - 1) and the rotation
 // (prefill_rot2_kernel's tasks, the workgroups after them) in one launch: both read only the picks of the launches
 // before, and neither waits for the other.
@@ -1197,6 +1229,7 @@ float* prefill_output(const gfr_fast_experts* fx) { return fx->out; }
 int prefill_item_rows(const gfr_fast_experts* fx, int rows, int bits) {
     return form_rows(window_form(fx, rows), bits);
 }
+constexpr int ROUTE_ONE_PICKS = 100;   // picks of a window up to which one launch routes, groups and rotates it
 hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_experts* w,
                                   const uint16_t* input, int input_stride, const float* logits, int rows, int routed,
                                   int topk, int* picks, float* weights, int* ids, int* count, int* members, int maxm,
@@ -1209,6 +1242,20 @@ hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr
         return hipErrorNotSupported;
     constexpr int WG = 512;                              // route_group measured the same at 512 and 1024 threads
     const int tasks = rows * (d.hidden / 256), grid = 1 + (tasks + WG / 64 - 1) / (WG / 64);
+    // Workgroup 0's eight waves route the rows eight at a time, 0.14 us a row at top-4 of 64, 0.27 at top-8 of 160 and
+    // 0.53 at GLM's top-8 of 288: past about 100 picks a launch that routes every row at once, ahead of the grouping and
+    // the rotation, costs less. A layer, one launch / two (us): hidden 2048, top-4 of 64: 20 rows 73.9 / 75.0, 32 rows
+    // 89.6 / 88.8, 100 rows 137 / 128, 220 rows 187 / 171; hidden 5120, top-8 of 160: 20 rows 254.6 / 255.3, 77 rows 501 /
+    // 494, 220 rows 680 / 638; hidden 4096, top-8 of 288: 20 rows 129 / 124, 100 rows 270 / 235, 220 rows 416 / 336.
+    if (rows * topk > ROUTE_ONE_PICKS) {
+        hipError_t e = launch_route(s, logits, rows, routed, topk, routed, picks, weights, bias, scale);
+        if (e != hipSuccess) return e;
+        group_small_rot_kernel<2><<<grid, WG, group_small_lds(rows, slots, routed + 1), s>>>(
+            picks, rows, slots, routed + 1, ids, count, members, maxm, prefill_item_rows(fx, rows, w->bits), fx->ucnt,
+            fx->items, fx->plan, w->experts, input, input_stride, w->suh_g, w->suh_u, fx->xg, fx->xu, d.hidden,
+            d.exl3_slots);
+        return hipGetLastError();
+    }
     route_group_rot_kernel<2><<<grid, WG, lds, s>>>(logits, rows, routed, topk, picks, weights, ids, count, members,
                                                     maxm, prefill_item_rows(fx, rows, w->bits), fx->ucnt, fx->items,
                                                     fx->plan, w->experts, RouteGate{bias, scale}, input, input_stride,

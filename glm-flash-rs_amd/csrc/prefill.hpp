@@ -28,8 +28,9 @@ hipError_t launch_group_large_rot(gfr_fast_experts* fx, hipStream_t s, const gfr
                                   const uint16_t* input, int input_stride, const int* picks, int rows, int slots,
                                   int E, uint32_t* bits, uint8_t* first, int* prefix, int* counts, int* ids,
                                   int* count, int* members, int maxm);
-// Route + group + item plan (launch_route_group's work) and prefill_run's input rotation in one launch, for a
-// window of the Moe path (the two input rotations apart); prefill_run then runs with planned and rotated. Returns
+// Route + group + item plan (launch_route_group's work) and prefill_run's input rotation in one launch, or for more
+// than a few rows in two (every row routed, then the rest), for a window of the Moe path (the two input rotations
+// apart); prefill_run then runs with planned and rotated. Returns
 // hipErrorNotSupported where the window does not fit the fused form (the caller then launches the parts).
 hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_experts* w,
                                   const uint16_t* input, int input_stride, const float* logits, int rows, int routed,

@@ -219,7 +219,9 @@ def test_prefill_rotation_bitexact(gfr, oracle, hidden, slots, rows, shared_x):
 @pytest.mark.parametrize("hidden,routed,topk,rows,glm", [
     (2048, 64, 4, 37, False),     # config 3's shape: softmax gate, 5 slots
     (1024, 288, 8, 9, True),      # the reference's router: GLM's biased sigmoid gate over 288 experts, 9 slots
-    (512, 16, 2, 256, False),     # the largest window of the route + group + rotation launch
+    (1024, 288, 8, 12, True),     # 96 picks: the most one launch routes, groups and rotates ...
+    (1024, 288, 8, 13, True),     # ... 104: a launch that routes, then one that groups and rotates
+    (512, 16, 2, 256, False),     # the largest window of those launches
     (512, 16, 2, 300, False),     # larger windows: the rotation rides on the grouping's scatter launch
     (1024, 288, 8, 260, True),    # ... with GLM's gate, full-K items
 ])
