@@ -133,9 +133,12 @@ def _ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+# The current stream's handle without a torch.cuda.Stream object around it: every run call asks for it.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _stream(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    return stream.cuda_stream if stream is not None else _raw_stream(torch.cuda.current_device())
 
 
 class _DeviceArray:
@@ -203,9 +206,24 @@ class Exl3Experts:
                 raise ValueError(f"{name}: {tuple(t.shape)} {t.dtype}, want {shape} {dtype} contiguous on GPU")
 
     def struct(self) -> "_Exl3Struct":
-        self.check()
-        return _Exl3Struct(self.experts, self.hidden, self.inter, self.bits, *(
-            _ptr(getattr(self, n)) for n in ("gt", "ut", "dt", "suh_g", "suh_u", "suh_d", "svh_g", "svh_u", "svh_d")))
+        # check()'s conditions on every call, without its table of names (a bs = 1 layer's three launches are submitted
+        # faster than that table is built); check() itself words the error
+        gt, ut, dt = self.gt, self.ut, self.dt
+        sg, su, sd, vg, vu, vd = self.suh_g, self.suh_u, self.suh_d, self.svh_g, self.svh_u, self.svh_d
+        E, D, N, b = gt.shape[0], sg.shape[1], sd.shape[1], self.bits
+        up, down, hid, mid = (E, D // 16, N // 16, 8 * b), (E, N // 16, D // 16, 8 * b), (E, D), (E, N)
+        i32, f16 = torch.int32, torch.float16
+        if not (gt.shape == up and ut.shape == up and dt.shape == down and sg.shape == hid and su.shape == hid
+                and vd.shape == hid and sd.shape == mid and vg.shape == mid and vu.shape == mid
+                and gt.dtype is i32 and ut.dtype is i32 and dt.dtype is i32 and sg.dtype is f16 and su.dtype is f16
+                and sd.dtype is f16 and vg.dtype is f16 and vu.dtype is f16 and vd.dtype is f16
+                and gt.is_contiguous() and ut.is_contiguous() and dt.is_contiguous() and sg.is_contiguous()
+                and su.is_contiguous() and sd.is_contiguous() and vg.is_contiguous() and vu.is_contiguous()
+                and vd.is_contiguous() and gt.is_cuda and ut.is_cuda and dt.is_cuda and sg.is_cuda and su.is_cuda
+                and sd.is_cuda and vg.is_cuda and vu.is_cuda and vd.is_cuda):
+            self.check()
+        return _Exl3Struct(E, D, N, b, gt.data_ptr(), ut.data_ptr(), dt.data_ptr(), sg.data_ptr(), su.data_ptr(),
+                           sd.data_ptr(), vg.data_ptr(), vu.data_ptr(), vd.data_ptr())
 
 
 class _Exl3Struct(ctypes.Structure):
@@ -262,9 +280,21 @@ class Fp8SharedWeights:
                 raise ValueError(f"{name}: want a contiguous tensor on the GPU")
 
     def struct(self) -> "_Fp8Struct":
-        self.check()
-        return _Fp8Struct(self.hidden, self.inter, *(_ptr(getattr(self, n)) for n in (
-            "gu", "gu_scale", "down", "down_scale", "gu_bf16", "down_bf16")))
+        gu, gs, down, ds, gu16, down16 = (self.gu, self.gu_scale, self.down, self.down_scale, self.gu_bf16,
+                                          self.down_bf16)
+        H, I = gu.shape[1], gu.shape[0] // 2
+        bf = torch.bfloat16
+        # check()'s conditions on every call, as in Exl3Experts.struct; check() itself words the error
+        copies = (gu16 is None and down16 is None) or (
+            gu16 is not None and down16 is not None and gu16.shape == (2 * I, H) and down16.shape == (H, I)
+            and gu16.dtype is bf and down16.dtype is bf and gu16.is_contiguous() and down16.is_contiguous()
+            and gu16.is_cuda and down16.is_cuda)
+        if not (copies and gu.shape == (2 * I, H) and gs.shape == (2 * I,) and down.shape == (H, I)
+                and ds.shape == (H,) and gs.dtype is bf and ds.dtype is bf and gu.element_size() == 1
+                and down.element_size() == 1 and gu.is_contiguous() and gs.is_contiguous() and down.is_contiguous()
+                and ds.is_contiguous() and gu.is_cuda and gs.is_cuda and down.is_cuda and ds.is_cuda):
+            self.check()
+        return _Fp8Struct(H, I, gu.data_ptr(), gs.data_ptr(), down.data_ptr(), ds.data_ptr(), _ptr(gu16), _ptr(down16))
 
 
 class _Fp8Struct(ctypes.Structure):
