@@ -116,52 +116,38 @@ __device__ __forceinline__ void decode_lane(const uint32_t (&w)[K], uint32_t pre
 
 
 // ---- the decode GEMV's dot: codebook words against activations, without the fp16 weight in between -------------
-// For one state s (16 bits, in half SEL of r), the masked codebook word m = (s * 0xCBAC1FED mod 2^32 & 0x8FFF8FFF) ^
+// For one state s (16 bits), the masked codebook word m = (s * 0xCBAC1FED mod 2^32 & 0x8FFF8FFF) ^
 // 0x3B603B60 (experts.rs:43-46) holds the two fp16 halves whose sum is the weight. The GEMV adds both halves times
 // the activation in one v_dot2_f32_f16 against the activation staged twice, (x, x): acc + x * m.lo + x * m.hi in
 // fp32. The reference rounds m.lo + m.hi to fp16 first; this sum keeps that rounding
-// out (a difference of at most half an fp16 ulp of each weight). Four VALU operations a weight at K = 4:
-//   v_and_b32 / v_lshrrev_b32   the state's half of r, alone in a register
-//   v_mul_lo_u32                s * 0xCBAC1FED mod 2^32
-//   v_bitop3                    mask, flip
-//   v_dot2_f32_f16              acc += x * m.lo + x * m.hi
-// Every constant is a VGPR operand (CodewordConsts): on gfx950 an SGPR or literal operand makes a VALU operation of
-// two issue passes where the all-VGPR v_and / v_lshrrev / v_bitop3 take one. Measured per decoded state and SIMD,
-// three waves a SIMD: 8.62 ns for the earlier form (v_pk_mul_lo_u16 + v_mad_u32_u16 with SGPR constants, SGPR mask),
-// 7.82 ns for this one. The other widths: v_pk_mul_lo_u16 (0, s * 0xCBAC) and v_mad_u32_u16 s * 0x1FED + that, then
-// the mask and the dot. (op_sel on the v_dot2 operands is not encodable on gfx950, hence the doubled activations.)
+// out (a difference of at most half an fp16 ulp of each weight). Four VALU operations a weight:
+//   v_and_b32 / v_lshrrev_b32 / v_bfe_u32   the state's 16 bits, alone in a register
+//   v_mul_lo_u32                            s * 0xCBAC1FED mod 2^32
+//   v_bitop3                                mask, flip
+//   v_dot2_f32_f16                          acc += x * m.lo + x * m.hi
+// and the window: one funnel shift holds two states at K = 2 and 4 (values 16 / K apart sit in its halves) and four at
+// K = 3 and 5 (3 K + 16 <= 31 bits). Isolating the state first takes one multiply where v_pk_mul_lo_u16 +
+// v_mad_u32_u16 (whose op_sel picks a half) take two: a bs = 1 layer at hidden 5120 measured 48.8 -> 44.8 us at K = 3,
+// 54.5 -> 50.6 at K = 5, 45.6 -> 45.1 at K = 2, same bits. At K = 4 every constant is a VGPR operand
+// (CodewordConsts): an SGPR or literal operand makes a VALU operation of two issue passes where the all-VGPR v_and /
+// v_lshrrev / v_bitop3 take one (per decoded state and SIMD, three waves a SIMD, 7.82 ns against 8.62 with SGPR
+// constants). At the other widths the two extra VGPRs cost a resident wave and the compiler places the constants
+// (measured 1-2 % slower with VGPR constants at K = 2, 3 and 5). (op_sel on the v_dot2 operands is not encodable on
+// gfx950, hence the doubled activations.)
 struct CodewordConsts {
     uint32_t lo16, mul, mask, flip;
 };
 // Made once per kernel: at K = 4 the asm hides the values, so the compiler keeps them in VGPRs and does not fold
-// them (the other widths' codeword does not read them).
+// them.
 template <int K>
 __device__ __forceinline__ CodewordConsts codeword_consts() {
     CodewordConsts c{0xffffu, 0xCBAC1FEDu, 0x8FFF8FFFu, 0x3B603B60u};
     if constexpr (K == 4) __asm__ volatile("" : "+v"(c.lo16), "+v"(c.mul), "+v"(c.mask), "+v"(c.flip));
     return c;
 }
-// K = 4 (config 2's width) takes the v_mul_lo_u32 form with VGPR constants; the other widths keep v_pk_mul_lo_u16 +
-// v_mad_u32_u16, whose op_sel picks the state's half without a mask (measured: the mul form is 2 % faster on
-// config 2's layer, and 1-2 % slower at K = 2 and 3, whose kernels lose a resident wave to its two extra VGPRs).
-template <int SEL, int K>
-__device__ __forceinline__ uint32_t codeword(uint32_t r, const CodewordConsts& c) {
-    uint32_t x;
-    if constexpr (K == 4) {
-        const uint32_t s = SEL == 0 ? (r & c.lo16) : (r >> 16);
-        x = s * c.mul;
-    } else {
-        uint32_t t;
-        if constexpr (SEL == 0) {
-            __asm__("v_pk_mul_lo_u16 %0, %1, %2 op_sel:[0,0] op_sel_hi:[0,1]" : "=v"(t) : "v"(r), "s"(0xCBAC0000u));
-            __asm__("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(x) : "v"(r), "s"(0x1FEDu), "v"(t));
-        } else {
-            __asm__("v_pk_mul_lo_u16 %0, %1, %2 op_sel:[1,0] op_sel_hi:[1,1]" : "=v"(t) : "v"(r), "s"(0xCBAC0000u));
-            __asm__("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(x) : "v"(r), "s"(0x1FEDu), "v"(t));
-        }
-        return (x & 0x8FFF8FFFu) ^ 0x3B603B60u;
-    }
-    return mask_flip(x, c.mask, c.flip);
+// The masked codebook word of a state.
+__device__ __forceinline__ uint32_t codeword(uint32_t s, const CodewordConsts& c) {
+    return mask_flip(s * c.mul, c.mask, c.flip);
 }
 // The lane's stream shifted right so that the window of value Q ends at bit 0, all 32 bits (bits 16-31: the 16
 // stream bits before the window).
@@ -173,7 +159,8 @@ __device__ __forceinline__ uint32_t lane_window32(const uint32_t (&w)[K], uint32
 }
 
 // Masked codebook words of the lane's 32 values, value order. K = 2 and 4: one 32-bit window holds the states of
-// values Q (low half) and Q - 16 / K (high half).
+// values Q (low half) and Q - 16 / K (high half); K = 3 and 5: the window of value Q | 3 holds its group of four, value
+// Q at bit (3 - Q % 4) K.
 template <int K, int Q>
 __device__ __forceinline__ void lane_word(const uint32_t (&w)[K], uint32_t prev, uint32_t (&m)[32],
                                           const CodewordConsts& c) {
@@ -181,11 +168,13 @@ __device__ __forceinline__ void lane_word(const uint32_t (&w)[K], uint32_t prev,
         constexpr int D = 16 / K;
         if constexpr (Q % (2 * D) >= D) {
             const uint32_t r = lane_window32<K, Q>(w, prev);
-            m[Q] = codeword<0, K>(r, c);
-            m[Q - D] = codeword<1, K>(r, c);
+            m[Q] = codeword(r & c.lo16, c);
+            m[Q - D] = codeword(r >> 16, c);
         }
     } else {
-        m[Q] = codeword<0, K>(lane_window<K, Q>(w, prev), c);
+        static_assert(3 * K + 16 <= 32, "four windows in one funnel word");
+        const uint32_t r = lane_window32<K, (Q | 3)>(w, prev);
+        m[Q] = codeword(Q % 4 == 3 ? r & c.lo16 : __builtin_amdgcn_ubfe(r, (3 - Q % 4) * K, 16), c);
     }
 }
 template <int K, int... Q>
