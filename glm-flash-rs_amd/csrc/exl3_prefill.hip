@@ -1135,6 +1135,15 @@ static hipError_t launch_gemm(Form f, int bits, dim3 grid, hipStream_t s, const 
     return hipGetLastError();
 }
 
+bool prefill_fits(const gfr_fast_experts* fx, const gfr_exl3_experts* w, int rows) {
+    const PrefillDims& d = fx->d;
+    const uint64_t P = (uint64_t)rows * d.slots, lim = 1ull << 32;
+    if ((P < (uint64_t)w->experts ? P : (uint64_t)w->experts) > (uint64_t)PF_MAXU) return false;
+    // the GEMM's direct loads address rows and trellis words by 32-bit byte offsets from their matrix
+    return P * d.hidden * 2 < lim && P * d.inter * 2 < lim &&
+           (uint64_t)w->experts * d.hidden * d.inter * w->bits / 8 < lim;
+}
+
 hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_experts* w, const uint16_t* input,
                        int input_stride, const int* picks, const int* ids, const int* count, const int* members,
                        int rows, int maxm, bool shared_x, const float* combine_weights, float* combine_out,
@@ -1142,15 +1151,9 @@ hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_exper
                        hipEvent_t shared_ready, bool rotated) {
     const PrefillDims& d = fx->d;
     if (combined) *combined = false;
-    if (w->bits < 2 || w->bits > 5) return hipErrorInvalidValue;
+    if (w->bits < 2 || w->bits > 5 || !prefill_fits(fx, w, rows)) return hipErrorInvalidValue;
     const int P = rows * d.slots;
     const int maxu = P < w->experts ? P : w->experts;
-    if (maxu > PF_MAXU) return hipErrorInvalidValue;
-    // the GEMM's direct loads address rows and trellis words by 32-bit byte offsets from their matrix
-    const uint64_t lim = 1ull << 32;
-    if ((uint64_t)P * d.hidden * 2 >= lim || (uint64_t)P * d.inter * 2 >= lim ||
-        (uint64_t)w->experts * d.hidden * d.inter * w->bits / 8 >= lim)
-        return hipErrorInvalidValue;
     hipError_t e;
     // rotated rows of every EXL3 pair (one copy when the two input rotations are the same)
     if (rotated) {

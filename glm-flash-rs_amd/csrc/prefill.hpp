@@ -14,6 +14,8 @@ struct PrefillDims {
 hipError_t prefill_create(gfr_fast_experts** out, int hidden, int inter, int slots, int exl3_slots, int experts,
                           int max_rows);
 PrefillDims prefill_dims(const gfr_fast_experts* fx);
+// The window and the weights are inside the GEMM's 32-bit offsets and plan (prefill_run refuses others).
+bool prefill_fits(const gfr_fast_experts* fx, const gfr_exl3_experts* w, int rows);
 hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_experts* w, const uint16_t* input,
                        int input_stride, const int* picks, const int* ids, const int* count, const int* members,
                        int rows, int maxm, bool shared_x, const float* combine_weights = nullptr,

@@ -140,7 +140,8 @@ float* gfr_moe_weights(const gfr_moe* m);        /* [rows][topk + 1] */
  * the prefill engine (windows above decode_rows), [rows * (topk + 1)][hidden] fp16 in the same pair order, matrix 0
  * (gate) or 1 (up). Windows of at most 256 rows rotate them in the route + group launch. Null for mat not 0 or 1. */
 uint16_t* gfr_moe_rotated(const gfr_moe* m, int mat);
-/* Windows of at most decode_rows rows run the decode engine (default 4, at most 64), larger ones the prefill engine.
+/* Windows of at most decode_rows rows run the decode engine (at most 64; default 4, fewer where hidden x inter x
+ * (topk + 1) passes 22 million weights, 1 from 45 million on), larger ones the prefill engine.
  * rows == 1 runs three launches: gate/up GEMV (router and input rotation fused), down GEMV (gate/up epilogue fused),
  * sum of the down parts + combine. */
 int gfr_moe_set_decode_rows(gfr_moe* m, int decode_rows);

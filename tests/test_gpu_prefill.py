@@ -348,3 +348,30 @@ def test_prefill_item_bodies(gfr, oracle, bits, form, hidden, inter):
     bound = 3 * 2.0 ** -8 * 150 / (80 * (inter / 2) ** 0.5)
     assert_rows_close(fx.output[:rows].cpu().numpy(), window_reference(oracle, w, x, picks_np).reshape(rows, hidden),
                       rel_rms=bound, what=f"{form} K={bits} {hidden}x{inter}")
+
+
+@pytest.mark.parametrize("hidden,inter,topk,limit", [(2560, 1536, 7, 2), (5120, 1536, 8, 1), (3072, 1536, 4, 3),
+                                                     (2048, 1536, 4, 4), (2560, 768, 7, 4)])
+def test_moe_small_windows_on_both_engines(gfr, oracle, hidden, inter, topk, limit):
+    """Windows on both sides of the engines' default border (from hidden x inter x slots): the prefill engine rotates its
+    rows, the decode engine leaves that probe alone; both give every token's output. A layer of at most 4 rows takes no
+    smaller border."""
+    import synth
+    E, bits = topk + 2, 4
+    w = synth.experts(E + 1, hidden, inter, bits, seed=800 + topk)
+    m = gfr.Moe(hidden, inter, E, topk, 5)
+    for rows in range(1, 6):
+        x, lg = synth.activations(rows, hidden, 810 + rows), synth.zipf_logits(rows, E, topk, 1.1, 820 + rows)
+        for mat in (0, 1):
+            m.rotated(mat, rows).zero_()
+        m.run(w, x, lg, rows)
+        torch.cuda.synchronize()
+        assert bool((m.rotated(0, rows) != 0).any()) == (rows > limit), rows
+        p, wt = oracle.route(lg.cpu().numpy(), topk, E)
+        y = window_reference(oracle, w, x, p)
+        want = np.einsum("rs,rsd->rd", wt.astype(np.float64), y.astype(np.float64))
+        # the decode engine multiplies unrounded codebook sums (within 1e-2 of the reference's fp16 weights)
+        assert_rows_close(m.output[:rows].cpu().numpy(), want, rel_rms=1e-2 if rows <= limit else 2e-3, what=f"{rows} rows")
+    small = gfr.Moe(hidden, inter, E, topk, 3)
+    with pytest.raises(gfr.GfrError):
+        small.set_decode_rows(0)
