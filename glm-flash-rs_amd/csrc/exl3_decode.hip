@@ -835,13 +835,22 @@ __global__ void __launch_bounds__(1024) down_finish_kernel(const float* __restri
 
 // gateup epilogue (exl3.cu:260-296): ordered split sums of gate and up, rotation, svh scales, GLM's limited SwiGLU
 // with its bf16 roundings, suh_d scale, rotation -> xd fp16. One wave a (pair, 128-column block).
+// FP8: workgroups x >= P run the layer's FP8 shared expert's down programs (a 16-column tile each).
+template <bool FP8>
 __global__ void __launch_bounds__(64) gateup_epilogue_kernel(const float* __restrict__ Z, const int* __restrict__ pick,
                                                               const uint16_t* __restrict__ svh_g,
                                                               const uint16_t* __restrict__ svh_u,
                                                               const uint16_t* __restrict__ suh_d,
                                                               uint16_t* __restrict__ xd, int P, int N, int SK,
-                                                              int slots, int exl3_slots, float limit, int pairs) {
+                                                              int slots, int exl3_slots, float limit, int pairs,
+                                                              const Fp8Args f, int rows) {
     const int p = blockIdx.x, blk = blockIdx.y;
+    if (FP8 && p >= P) {
+        const int nt = (p - P) * gridDim.y + blk;
+        if (nt < f.hidden / 16)
+            fp8_down_program<8>(f.w, f.s, f.x, rows, 0, f.inter, nt, threadIdx.x, f.out, f.hidden);
+        return;
+    }
     const int row = p / slots, slot = p % slots;
     if (slot >= exl3_slots) return;
     const int lane = threadIdx.x;
@@ -1155,9 +1164,17 @@ hipError_t launch_down_finish(hipStream_t s, const float* Zd, const int* pick, c
 
 hipError_t launch_gateup_epilogue(hipStream_t s, const float* Z, const int* pick, const uint16_t* svh_g,
                                   const uint16_t* svh_u, const uint16_t* suh_d, uint16_t* xd, int P, int N, int SK,
-                                  int slots, int exl3_slots, float limit, bool pair_order) {
-    gateup_epilogue_kernel<<<dim3(P, N / 128), 64, 0, s>>>(Z, pick, svh_g, svh_u, suh_d, xd, P, N, SK, slots,
-                                                           exl3_slots, limit, pair_order ? 1 : 0);
+                                  int slots, int exl3_slots, float limit, bool pair_order, const Fp8Shared* fp8,
+                                  int rows) {
+    Fp8Args f{};
+    int x = P;
+    if (fp8) {
+        f = Fp8Args{fp8->d_w, fp8->d_s, fp8->act, nullptr, nullptr, fp8->out, fp8->hidden, fp8->inter};
+        x += (fp8->hidden / 16 + N / 128 - 1) / (N / 128);
+    }
+    auto go = fp8 ? gateup_epilogue_kernel<true> : gateup_epilogue_kernel<false>;
+    go<<<dim3(x, N / 128), 64, 0, s>>>(Z, pick, svh_g, svh_u, suh_d, xd, P, N, SK, slots, exl3_slots, limit,
+                                       pair_order ? 1 : 0, f, rows);
     return hipGetLastError();
 }
 

@@ -30,6 +30,7 @@
 #include "launch.hpp"
 #include "prefill.hpp"
 #include "grouping_body.hpp"
+#include "shared_fp8.hpp"
 
 namespace gfr {
 
@@ -359,12 +360,22 @@ __global__ void __launch_bounds__(256) prefill_rot2_kernel(const uint16_t* __res
                     out1, K, row, bp, slots, exl3_slots);
 }
 
+// The layer's FP8 shared expert in a window of at most 16 rows: its gate/up programs (8 intermediate indices a
+// workgroup of 8 waves, one K slice each) are workgroups 1 .. inter / 8 of the launches below, which need nothing of each
+// other; its down programs ride on the gate/up epilogue's launch. Its own two launches took 8.0 + 4.0 us next to these
+// launches' 12.6 and 4.7 (12 rows, 288 experts): a layer 93 -> 85 us.
+__device__ __forceinline__ void fp8_gu_workgroup(const Fp8Args& f, int rows) {
+    __shared__ Fp8Part part;
+    fp8_gu_program<8, FP8_SLICES, 8>(f.w, f.s, f.x, f.hidden, rows, 0, f.hidden, f.inter, blockIdx.x - 1,
+                                     threadIdx.x >> 6, threadIdx.x & 63, part, f.gu, f.act);
+}
+
 // Route + group + item plan and the rotation of every EXL3 pair in one launch, for the windows route_group_kernel
 // takes (K / 128 even). Workgroup 0 does route_group_kernel's work (route_group_body; its dynamic LDS); the others
 // take prefill_rot2_kernel's tasks, a wave's task routing its token with the same router (route_load / route_pick on
 // the same logits, so the same picks as workgroup 0 writes) while its token loads are in flight. Nothing of one
 // part waits for the other.
-template <int MATS>
+template <int MATS, bool FP8>
 __global__ void __launch_bounds__(512) route_group_rot_kernel(const float* __restrict__ logits, int rows, int routed,
                                                               int topk, int* __restrict__ picks,
                                                               float* __restrict__ weights, int* __restrict__ ids,
@@ -376,7 +387,7 @@ __global__ void __launch_bounds__(512) route_group_rot_kernel(const float* __res
                                                               const uint16_t* __restrict__ suh0,
                                                               const uint16_t* __restrict__ suh1,
                                                               uint16_t* __restrict__ out0, uint16_t* __restrict__ out1,
-                                                              int K, int exl3_slots) {
+                                                              int K, int exl3_slots, const Fp8Args f) {
     extern __shared__ uint32_t lds[];
     __shared__ __attribute__((aligned(16))) int scan_scratch[16];
     if (blockIdx.x == 0) {
@@ -384,7 +395,9 @@ __global__ void __launch_bounds__(512) route_group_rot_kernel(const float* __res
                          plan_ucnt, plan_items, plan, plan_E, gate);
         return;
     }
-    const int task = (blockIdx.x - 1) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int fwg = FP8 ? f.inter / 8 : 0;
+    if (FP8 && (int)blockIdx.x <= fwg) return fp8_gu_workgroup(f, rows);
+    const int task = ((int)blockIdx.x - 1 - fwg) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int KP = K / 256, row = task / KP, bp = task % KP;
     if (row >= rows) return;
     const int lane = threadIdx.x & 63;
@@ -402,7 +415,7 @@ __global__ void __launch_bounds__(512) route_group_rot_kernel(const float* __res
 // group_small_kernel's work (with the item plan) in workgroup 0 and the rotation's tasks in the others, for windows
 // whose picks are routed: launch_route_group_rot's second launch where one workgroup's routing of every row would
 // outlast the rest.
-template <int MATS>
+template <int MATS, bool FP8>
 __global__ void __launch_bounds__(512) group_small_rot_kernel(const int* __restrict__ picks, int rows, int slots, int E,
                                                               int* __restrict__ ids, int* __restrict__ count,
                                                               int* __restrict__ members, int maxm, int bm,
@@ -412,7 +425,7 @@ __global__ void __launch_bounds__(512) group_small_rot_kernel(const int* __restr
                                                               const uint16_t* __restrict__ suh0,
                                                               const uint16_t* __restrict__ suh1,
                                                               uint16_t* __restrict__ out0, uint16_t* __restrict__ out1,
-                                                              int K, int exl3_slots) {
+                                                              int K, int exl3_slots, const Fp8Args f) {
     extern __shared__ uint32_t lds[];
     __shared__ __attribute__((aligned(16))) int scan_scratch[16];
     if (blockIdx.x == 0) {
@@ -424,7 +437,9 @@ __global__ void __launch_bounds__(512) group_small_rot_kernel(const int* __restr
         return;
     }
     const int lane = threadIdx.x & 63;
-    const int task = (blockIdx.x - 1) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int fwg = FP8 ? f.inter / 8 : 0;
+    if (FP8 && (int)blockIdx.x <= fwg) return fp8_gu_workgroup(f, rows);
+    const int task = ((int)blockIdx.x - 1 - fwg) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int KP = K / 256, row = task / KP, bp = task % KP;
     if (row >= rows) return;
     rot2_task<MATS>(x, x_stride, [&] { return lane < exl3_slots ? picks[row * slots + lane] : 0; }, suh0, suh1, out0,
@@ -1148,7 +1163,7 @@ hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_exper
                        int input_stride, const int* picks, const int* ids, const int* count, const int* members,
                        int rows, int maxm, bool shared_x, const float* combine_weights, float* combine_out,
                        bool* combined, bool planned, const float* combine_shared, int shared_stride,
-                       hipEvent_t shared_ready, bool rotated) {
+                       hipEvent_t shared_ready, bool rotated, const Fp8Shared* fp8) {
     const PrefillDims& d = fx->d;
     if (combined) *combined = false;
     if (w->bits < 2 || w->bits > 5 || !prefill_fits(fx, w, rows)) return hipErrorInvalidValue;
@@ -1204,7 +1219,7 @@ hipError_t prefill_run(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_exper
         a.x0 = fx->xg; a.x1 = shared_x ? fx->xg : fx->xu; a.t0 = w->gt; a.t1 = w->ut; a.Kin = d.hidden; a.N = d.inter;
         if ((e = launch_gemm<2>(form, w->bits, dim3(max_items * (d.inter / 128) * skg), s, a)) != hipSuccess) return e;
         if ((e = launch_gateup_epilogue(s, fx->zgu, picks, w->svh_g, w->svh_u, w->suh_d, fx->xd, P, d.inter, skg,
-                                        d.slots, d.exl3_slots, 10.f, true)) != hipSuccess)
+                                        d.slots, d.exl3_slots, 10.f, true, fp8, rows)) != hipSuccess)
             return e;
         a.sk = skd; a.z = fx->zd;
         a.x0 = fx->xd; a.x1 = fx->xd; a.t0 = w->dt; a.t1 = w->dt; a.Kin = d.inter; a.N = d.hidden;
@@ -1232,19 +1247,30 @@ float* prefill_output(const gfr_fast_experts* fx) { return fx->out; }
 int prefill_item_rows(const gfr_fast_experts* fx, int rows, int bits) {
     return form_rows(window_form(fx, rows), bits);
 }
+// The windows launch_route_group_rot takes.
+static bool fused_window(const gfr_fast_experts* fx, const gfr_exl3_experts* w, int rows, int routed, int topk) {
+    const PrefillDims& d = fx->d;
+    return rows >= 1 && rows <= GROUP_SMALL_ROWS && rows <= d.max_rows && routed + 1 <= 1024 && topk + 1 == d.slots &&
+           route_group_lds(rows, topk + 1, routed + 1) <= GROUP_LDS_MAX && (d.hidden / 128) % 2 == 0 && w->bits >= 2 &&
+           w->bits <= 5;
+}
+bool prefill_takes_fp8(const gfr_fast_experts* fx, const gfr_exl3_experts* w, int rows, int routed, int topk) {
+    return rows <= 16 && fused_window(fx, w, rows, routed, topk) && window_form(fx, rows) == Form::SPLIT &&
+           route_group_lds(rows, topk + 1, routed + 1) + sizeof(Fp8Part) <= GROUP_LDS_MAX;
+}
 constexpr int ROUTE_ONE_PICKS = 100;   // picks of a window up to which one launch routes, groups and rotates it
 hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_experts* w,
                                   const uint16_t* input, int input_stride, const float* logits, int rows, int routed,
                                   int topk, int* picks, float* weights, int* ids, int* count, int* members, int maxm,
-                                  const float* bias, float scale) {
+                                  const float* bias, float scale, const Fp8Shared* fp8) {
     const PrefillDims& d = fx->d;
     const int slots = topk + 1;
     const size_t lds = route_group_lds(rows, slots, routed + 1);
-    if (rows < 1 || rows > GROUP_SMALL_ROWS || rows > d.max_rows || routed + 1 > 1024 || slots != d.slots ||
-        lds > GROUP_LDS_MAX || (d.hidden / 128) % 2 || w->bits < 2 || w->bits > 5)
-        return hipErrorNotSupported;
+    if (!fused_window(fx, w, rows, routed, topk)) return hipErrorNotSupported;
+    Fp8Args f{};
+    if (fp8) f = Fp8Args{fp8->gu_w, fp8->gu_s, input, fp8->gu, fp8->act, nullptr, fp8->hidden, fp8->inter};
     constexpr int WG = 512;                              // route_group measured the same at 512 and 1024 threads
-    const int tasks = rows * (d.hidden / 256), grid = 1 + (tasks + WG / 64 - 1) / (WG / 64);
+    const int tasks = rows * (d.hidden / 256), grid = 1 + (fp8 ? f.inter / 8 : 0) + (tasks + WG / 64 - 1) / (WG / 64);
     // Workgroup 0's eight waves route the rows eight at a time, 0.14 us a row at top-4 of 64, 0.27 at top-8 of 160 and
     // 0.53 at GLM's top-8 of 288: past about 100 picks a launch that routes every row at once, ahead of the grouping and
     // the rotation, costs less. A layer, one launch / two (us): hidden 2048, top-4 of 64: 20 rows 73.9 / 75.0, 32 rows
@@ -1253,16 +1279,18 @@ hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr
     if (rows * topk > ROUTE_ONE_PICKS) {
         hipError_t e = launch_route(s, logits, rows, routed, topk, routed, picks, weights, bias, scale);
         if (e != hipSuccess) return e;
-        group_small_rot_kernel<2><<<grid, WG, group_small_lds(rows, slots, routed + 1), s>>>(
+        auto go = fp8 ? group_small_rot_kernel<2, true> : group_small_rot_kernel<2, false>;
+        go<<<grid, WG, group_small_lds(rows, slots, routed + 1), s>>>(
             picks, rows, slots, routed + 1, ids, count, members, maxm, prefill_item_rows(fx, rows, w->bits), fx->ucnt,
             fx->items, fx->plan, w->experts, input, input_stride, w->suh_g, w->suh_u, fx->xg, fx->xu, d.hidden,
-            d.exl3_slots);
+            d.exl3_slots, f);
         return hipGetLastError();
     }
-    route_group_rot_kernel<2><<<grid, WG, lds, s>>>(logits, rows, routed, topk, picks, weights, ids, count, members,
-                                                    maxm, prefill_item_rows(fx, rows, w->bits), fx->ucnt, fx->items,
-                                                    fx->plan, w->experts, RouteGate{bias, scale}, input, input_stride,
-                                                    w->suh_g, w->suh_u, fx->xg, fx->xu, d.hidden, d.exl3_slots);
+    auto go = fp8 ? route_group_rot_kernel<2, true> : route_group_rot_kernel<2, false>;
+    go<<<grid, WG, lds, s>>>(logits, rows, routed, topk, picks, weights, ids, count, members, maxm,
+                             prefill_item_rows(fx, rows, w->bits), fx->ucnt, fx->items, fx->plan, w->experts,
+                             RouteGate{bias, scale}, input, input_stride, w->suh_g, w->suh_u, fx->xg, fx->xu, d.hidden,
+                             d.exl3_slots, f);
     return hipGetLastError();
 }
 

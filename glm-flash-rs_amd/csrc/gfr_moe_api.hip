@@ -542,7 +542,7 @@ int moe_run(gfr_moe* m, hipStream_t stream, const gfr_exl3_experts* w, const uin
     bool planned = false, rotated = false;
     if ((e = gfr::launch_route_group_rot(m->pre, stream, w, input, m->hidden, logits, rows, m->routed, m->topk,
                                          m->picks, m->weights, g->ids, g->count, g->members, g->max_rows,
-                                         m->route_bias, m->route_scale)) == hipSuccess) {
+                                         m->route_bias, m->route_scale, fp8)) == hipSuccess) {
         // route + group + item plan and the input rotation in one launch
         planned = rotated = true;
     } else if (e != hipErrorNotSupported) {
@@ -589,7 +589,7 @@ int moe_run(gfr_moe* m, hipStream_t stream, const gfr_exl3_experts* w, const uin
     bool combined = false;
     if ((e = gfr::prefill_run(m->pre, stream, w, input, m->hidden, m->picks, g->ids, g->count, g->members, rows,
                               g->max_rows, false, m->weights, m->out, &combined, planned, shared, shared_stride,
-                              shared_ready, rotated)) != hipSuccess)
+                              shared_ready, rotated, fp8)) != hipSuccess)
         return hip_fail(e, "prefill run");
     if (!combined && shared_ready && (e = hipStreamWaitEvent(stream, shared_ready, 0)) != hipSuccess)
         return hip_fail(e, "wait for the shared expert");
@@ -836,14 +836,18 @@ int gfr_shared_fp8_destroy(gfr_shared_fp8* sh) {
 namespace {
 // The layer with its FP8 shared expert. A one-token window whose launches have the shared slot's workgroups (the
 // grid's last unit exists: the weights hold at least `slots` experts) runs the shared expert inside the gate/up and
-// down launches (three launches in all); other windows run its two launches first.
+// down launches (three launches in all), a prefill-engine window of at most 16 rows inside its route + group + rotation
+// and gate/up epilogue launches; other windows run its two launches first.
 int moe_run_fp8(gfr_moe* m, hipStream_t stream, const gfr_exl3_experts* w, const uint16_t* input,
                 const float* logits, const gfr_fp8_shared_weights* sw, int rows) {
     if (rows <= 0 || rows > m->max_rows) return fail(GFR_EINVAL, "rows %d outside 1..%d", rows, m->max_rows);
     if (!w || !input) return fail(GFR_EINVAL, "null weights or input");
     if (!al16(input)) return fail(GFR_EINVAL, "input rows must be 16-byte aligned");
-    const bool fused = rows == 1 && rows <= m->decode_rows && w->experts >= m->slots &&
-                       gfr::gemv_gateup_splits(m->hidden) <= 16;
+    // (the weights' other checks follow in moe_run, before any launch)
+    const bool fused = rows <= m->decode_rows
+                           ? rows == 1 && w->experts >= m->slots && gfr::gemv_gateup_splits(m->hidden) <= 16
+                           : w->hidden == m->hidden && w->inter == m->inter && gfr::prefill_fits(m->pre, w, rows) &&
+                                 gfr::prefill_takes_fp8(m->pre, w, rows, m->routed, m->topk);
     if (!fused) {
         int rc = shared_fp8_run(m->sfp8, stream, sw, input, m->hidden, rows, m->shared_out, m->hidden);
         if (rc) return rc;

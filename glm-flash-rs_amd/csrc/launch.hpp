@@ -98,7 +98,9 @@ hipError_t launch_down_finish(hipStream_t s, const float* Zd, const int* pick, c
 // pair_order: xd in the MFMA path's pair order (x[m + 8], x[m] within each 16-value tile) instead of k order
 hipError_t launch_gateup_epilogue(hipStream_t s, const float* Z, const int* pick, const uint16_t* svh_g,
                                   const uint16_t* svh_u, const uint16_t* suh_d, uint16_t* xd, int P, int N, int SK,
-                                  int slots, int exl3_slots, float limit, bool pair_order = false);
+                                  int slots, int exl3_slots, float limit, bool pair_order = false,
+                                  const Fp8Shared* fp8 = nullptr, int rows = 0);
+// fp8: the FP8 shared expert's down programs over its act rows (at most 16) in workgroups of the same launch
 hipError_t launch_down_epilogue(hipStream_t s, const float* Z, const int* pick, const uint16_t* svh_d, float* y,
                                 int P, int D, int SK, int slots, int exl3_slots);
 

@@ -232,6 +232,52 @@ def test_moe_run_fp8_one_token_forms(gfr, oracle, routed, topk, H, I):
         assert torch.equal(m.output[:1], got)
 
 
+@pytest.mark.parametrize("routed,topk,H,I,rows", [
+    (16, 4, 512, 256, 5),        # 32 down tiles, two a grid column
+    (16, 4, 512, 768, 16),       # six a column: the last column's tail is idle; 16 rows: a full tile
+    (16, 4, 512, 768, 17),       # the first window past the tile: its own launches
+    (12, 4, 1024, 256, 1),       # one row through the prefill engine
+    (40, 8, 1024, 256, 12),      # 96 picks: one launch routes, groups and rotates
+    (40, 8, 1024, 256, 13),      # 104 picks: two
+    (1000, 4, 512, 256, 7)])     # many experts: the grouping's LDS next to the program's
+def test_moe_run_fp8_window_forms(gfr, routed, topk, H, I, rows):
+    """Windows of the prefill engine with the FP8 shared expert: up to 16 rows ride on the layer's launches. The bytes
+    are those of gfr_moe_run_shared fed with gfr_shared_fp8's output (the same programs: no tolerance), eagerly, on
+    another window after it, and in every replay of a captured graph."""
+    import synth
+    w = synth.experts(routed, H, I, BITS, seed=routed)
+    sw1 = synth.fp8_shared(H, I, seed=routed + 1)
+    m = gfr.Moe(H, I, routed, topk, 20, shared_exl3=False)
+    m2 = gfr.Moe(H, I, routed, topk, 20, shared_exl3=False)
+    for mm in (m, m2):
+        mm.set_decode_rows(0)
+    x = lg = want = None
+    for seed in (2, 3):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        x = torch.randn((rows, H), generator=g, device="cuda").to(torch.bfloat16)
+        lg = synth.logits(rows, routed, seed + 10)
+        m.run_fp8(w, x, lg, sw1, rows)
+        shared = gfr.SharedFp8(H, I, rows).run(sw1, x, rows)
+        m2.run(w, x, lg, rows, shared=shared)
+        torch.cuda.synchronize()
+        want = m2.output[:rows].clone()
+        assert torch.equal(m.shared_output[:rows], shared)
+        assert torch.equal(m.output[:rows], want)
+    s = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(graph, stream=s):
+            m.run_fp8(w, x, lg, sw1, rows, stream=s)
+    for _ in range(3):
+        m.output.zero_()
+        m.shared_output.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(m.output[:rows], want)
+
+
 # ---- the prefill form (prefill.rs:55-150, batch.rs:1183-1195): bf16 weight copies and library GEMMs -----------------
 @pytest.fixture(scope="module")
 def sw_prepared():
