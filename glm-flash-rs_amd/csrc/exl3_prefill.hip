@@ -13,7 +13,7 @@
 //     (16 n x 8 k) once k is taken in the pair order of exl3_format.hpp (pair_row); the token rows (B operand) are
 //     staged in LDS in that same order, so no weight ever goes through LDS and none is decoded twice in a workgroup.
 //   * workgroup = 4 waves, a tile of BM member rows of one expert x 128 (gate/up: both matrices) or 256 (down)
-//     output columns, two workgroups a CU; each wave owns 64 columns x BM rows (4 BM / 16 MFMA 16x16 accumulators),
+//     output columns, two workgroups a CU (three where items are short, see PF_FEW); each wave owns 64 columns x BM rows (4 BM / 16 MFMA 16x16 accumulators),
 //     K in steps of 32, multi-stage direct-to-LDS staging and a register pipeline (next step's decode during this
 //     step's MFMAs). BM = 176 for K = 4: the trellis decode (VALU) is amortised over more rows, an expert of 512
 //     members takes 3 passes instead of 4, and 244 VGPRs and two workgroups' stages (2 x 80.6 KB) still fit.

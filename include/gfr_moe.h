@@ -138,7 +138,7 @@ int32_t* gfr_moe_picks(const gfr_moe* m);        /* [rows][topk + 1] */
 float* gfr_moe_weights(const gfr_moe* m);        /* [rows][topk + 1] */
 /* Parity probe, no reference counterpart (as gfr_fast_experts_rotated): the rotated input rows of the last run on
  * the prefill engine (windows above decode_rows), [rows * (topk + 1)][hidden] fp16 in the same pair order, matrix 0
- * (gate) or 1 (up). Windows of at most 256 rows rotate them in the route + group launch. Null for mat not 0 or 1. */
+ * (gate) or 1 (up). Windows of at most 256 rows rotate them in the grouping's launch. Null for mat not 0 or 1. */
 uint16_t* gfr_moe_rotated(const gfr_moe* m, int mat);
 /* Windows of at most decode_rows rows run the decode engine (at most 64; default 4, fewer where hidden x inter x
  * (topk + 1) passes 22 million weights, 1 from 45 million on), larger ones the prefill engine.
@@ -204,7 +204,8 @@ uint16_t* gfr_shared_fp8_act(const gfr_shared_fp8* sh);
 int gfr_shared_fp8_destroy(gfr_shared_fp8* sh);
 /* Moe::run_prefetched with its FP8 shared expert (moe.rs:66-182), for a layer made with gfr_moe_create_shared(...,
  * shared_exl3 = 0) and hidden a multiple of 512: the shared expert into the layer's own buffer
- * (gfr_moe_shared_output, [max_rows][hidden] fp32), then gfr_moe_run_shared with it. _router_fp8 computes the router
+ * (gfr_moe_shared_output, [max_rows][hidden] fp32), then gfr_moe_run_shared with it, in the same launches where these
+ * have room (one token; up to 16 rows on the prefill engine). _router_fp8 computes the router
  * logits first, as gfr_moe_run_router. Input rows [rows][hidden] bf16, 16-byte aligned. */
 int gfr_moe_run_fp8(gfr_moe* m, hipStream_t stream, const gfr_exl3_experts* w, const uint16_t* input,
                     const float* logits, const gfr_fp8_shared_weights* sw, int rows);
