@@ -611,10 +611,12 @@ __device__ __forceinline__ h8_t a_fragment(const uint32_t (&wd)[4], const uint32
 // all lanes active. Written as inline asm: the compiler treats its builtin as an LDS store of unknown address and puts
 // s_waitcnt vmcnt(0) before every later LDS read, which drains the whole load pipeline each step; here the kernels wait
 // for their stages themselves (wait_vmcnt), and loads complete in order, so any wait the compiler adds for its own loads
-// only waits longer.
+// only waits longer. The base goes through vcc by a scalar move: a VMEM instruction may read an SGPR that a VALU
+// instruction wrote (the v_readlane of a spilled base, a v_readfirstlane) only five wait states later, and the compiler,
+// which does not look into the asm, keeps no such distance; scalar instructions wait for VALU writes by themselves.
 __device__ __forceinline__ void load_lds16_s(uint64_t sbase, uint32_t voff, uint32_t m0, uint64_t mask) {
-    __asm__ volatile("s_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1"
-                     :: "v"(voff), "s"(sbase), "{m0}"(m0), "s"(mask) : "memory");
+    __asm__ volatile("s_mov_b64 exec, %3\n\ts_mov_b64 vcc, %1\n\tglobal_load_lds_dwordx4 %0, vcc\n\ts_mov_b64 exec, -1"
+                     :: "v"(voff), "s"(sbase), "{m0}"(m0), "s"(mask) : "memory", "vcc");
 }
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
     // readfirstlane returns int: through uint32_t, so that the low word is not sign-extended into the high one
