@@ -1109,26 +1109,26 @@ hipError_t prefill_create(gfr_fast_experts** out, int hidden, int inter, int slo
 
 PrefillDims prefill_dims(const gfr_fast_experts* fx) { return fx->d; }
 
-// The window's form, from its pairs P and the engine's experts E (the same rule for the plan and the launches):
+// The window's form, from its pairs P (every slot's, also those of a shared expert that is not EXL3) and the engine's
+// experts E (the same rule for the plan and the launches):
 //   SPLIT  split-K programs: windows whose full-K programs would leave CUs idle behind a few long ones;
 //   FEW    full-K items of up to PF_FEW rows, three workgroups a CU;
 //   LARGE  full-K items of pf_bm_for rows, two a CU: each decoded weight feeds more rows.
-// Up to PF_SPLIT_PAIRS pairs, FEW needs some rows an expert and gate/up programs for two rounds of 768 (us a layer,
-// split / few): hidden 5120, 160 + 1 experts, top-8: 64 rows 462 / 485, 77 rows (K = 3) 513 / 528, 100 rows 579 / 580
-// (K = 3) and 658 / 647 (uniform), 150 rows 711 / 656, 220 rows (K = 2) 773 / 685; fewer programs: hidden 2048, 64 + 1,
-// top-4, 300 rows 179 / 197 (uniform) and 200 / 193, hidden 4096, 288 experts, top-8, inter 512, 220 rows (K = 2) 412 /
-// 415. From PF_FEW_MEAN rows an expert LARGE wins where an expert's rows fit one of its passes (us a layer, few /
-// large): 16 (512 rows, 288 experts) 429 / 502; 77 (1000 rows, hidden 2048) 248 / 323; 84 (1500 rows, hidden 5120,
-// K = 3) 1405 / 1491; 94 (3000 rows, 288 experts) 979 / 1031; 112 (2000 rows, hidden 5120, uniform) 1798 / 1589; 630
-// (8192 rows, hidden 2048) 1323 / 1181.
+// FEW and LARGE add a sum's products in the same order and share the epilogue, so the border between them moves no bit.
+// SPLIT's sums and epilogue are others: at a shape that has it, every window of up to PF_SPLIT_PAIRS pairs runs it,
+// whatever FEW measures there (us a layer, split / few; hidden 5120, 160 + 1 experts, top-8: 64 rows 462 / 485, 100 rows
+// uniform 658 / 647, 150 rows 711 / 656, 220 rows K = 2 773 / 685), so that a row's bytes do not depend on how many
+// others an expert has. FEW against LARGE (us a layer, few / large): 16 pairs an expert (512 rows, 288 experts) 429 /
+// 502; 77 (1000 rows, hidden 2048) 248 / 323; 84 (1500 rows, hidden 5120, K = 3) 1405 / 1491; 94 (3000 rows, 288 experts)
+// 979 / 1031; 112 (2000 rows, hidden 5120, uniform) 1798 / 1589; 630 (8192 rows, hidden 2048) 1323 / 1181. Near the
+// border the popularity's skew decides (FP8 shared expert, K = 4): 128 (4096 rows, 288 experts) uniform 1156 / 1113,
+// Zipf(1.1) 1148 / 1181; 100 (1280 rows of 64) uniform 300 / 289, Zipf(1.1) 311 / 366.
 constexpr int PF_FEW_MEAN = 100;
 enum class Form { SPLIT, FEW, LARGE };
 static Form window_form(const gfr_fast_experts* fx, int rows) {
-    const int P = rows * fx->d.slots, E = fx->d.experts;
-    const int programs = (fx->d.inter / 128) * ((P < E ? P : E) + P / PF_FEW);
-    const bool many = P >= 6 * E && programs >= 2 * 3 * 256;
-    if (fx->zgu && P <= PF_SPLIT_PAIRS && !many) return Form::SPLIT;
-    return P < PF_FEW_MEAN * E ? Form::FEW : Form::LARGE;
+    const int P = rows * fx->d.slots;
+    if (fx->zgu && P <= PF_SPLIT_PAIRS) return Form::SPLIT;
+    return P < PF_FEW_MEAN * fx->d.experts ? Form::FEW : Form::LARGE;
 }
 static int form_rows(Form f, int bits) {
     return f == Form::SPLIT ? PF_SPLIT_BM : f == Form::FEW ? PF_FEW : pf_bm_for(bits);

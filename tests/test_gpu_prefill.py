@@ -350,6 +350,34 @@ def test_prefill_item_bodies(gfr, oracle, bits, form, hidden, inter):
                       rel_rms=bound, what=f"{form} K={bits} {hidden}x{inter}")
 
 
+@pytest.mark.parametrize("bits", [3, 4])
+def test_split_windows_do_not_depend_on_the_window(gfr, bits):
+    """Windows of up to 2048 pairs at a shape with the split-K programs run those, however many rows an expert has and
+    however many programs: a pair's output is the same bytes in a window of 256 rows (2048 pairs, 17 rows an expert) and
+    of 100 rows (6 an expert) as in one of 9 rows."""
+    import synth
+    E, hidden, inter, slots, rows = 120, 2048, 1536, 8, 256
+    w = synth.experts(E, hidden, inter, bits, seed=700 + bits)
+    x = synth.activations(rows, hidden, 701)
+    rng = np.random.default_rng(bits)
+    picks = torch.from_numpy(np.stack([rng.permutation(E)[:slots] for _ in range(rows)]).astype(np.int32)).cuda()
+    g = gfr.Grouping(E, slots, rows)
+    fx = gfr.FastExperts(hidden, inter, slots, slots, E, rows)
+
+    def window(r0, n):
+        p = picks[r0:r0 + n].contiguous()
+        g.run(p, n)
+        fx.run(w, x[r0:r0 + n].contiguous(), p, g.ids, g.count, g.members, n, rows, shared_x=False)
+        return fx.output[:n * slots].view(n, slots, hidden).clone()
+
+    small = torch.cat([window(r, min(9, rows - r)) for r in range(0, rows, 9)])
+    for n in (100, 256):
+        got = window(0, n)
+        assert torch.isfinite(got).all()
+        diff = (got != small[:n]).any(dim=2).any(dim=1).sum().item()
+        assert diff == 0, f"{diff} of {n} rows differ between a window of {n} rows and windows of 9"
+
+
 @pytest.mark.parametrize("hidden,inter,topk,limit", [(2560, 1536, 7, 2), (5120, 1536, 8, 1), (3072, 1536, 4, 3),
                                                      (2048, 1536, 4, 4), (2560, 768, 7, 4)])
 def test_moe_small_windows_on_both_engines(gfr, oracle, hidden, inter, topk, limit):
