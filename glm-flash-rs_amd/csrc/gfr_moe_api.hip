@@ -99,7 +99,6 @@ struct gfr_linear {
 
 struct gfr_moe {
     int hidden, inter, routed, topk, slots, max_rows, decode_rows;
-    int decode_most;           // windows up to this many rows run on the decode engine where the prefill engine cannot
     float* weights;
     int* picks;
     float* out;
@@ -419,26 +418,6 @@ int gfr_fast_experts_destroy(gfr_fast_experts* fx) {
 }
 
 // ---- one MoE layer ----------------------------------------------------------------------------------------------
-}  // extern "C"
-namespace {
-constexpr int MOE_DECODE_ROWS = 4;
-// The largest window the decode engine takes by default, from the weights a token meets in one of its matrices: its GEMV
-// reads each expert's trellis for at most a few rows, in programs that each build their activations; the split-K programs
-// decode once for 16 rows and pay two more launches. Measured (us a layer, decode / prefill engine, Zipf(1.1), K = 4):
-//   15.7 M (hidden 2048, inter 1536, 5 slots)  3 rows 41.1 / 44.8   4 rows 50.9 / 52.9   5 rows 60.6 / 52.9
-//   18.9 M (4096, 512, 9 slots, 288 experts)   3 rows 54.8 / 64.9   4 rows 65.5 / 64.9   5 rows 85.6 / 67.0
-//   23.6 M (3072, 1536, 5)                     3 rows 51.5 / 52.7   4 rows 65.6 / 53.3
-//   37.7 M (4096, 1024, 9)                     2 rows 51.0 / 56.0   3 rows 67.2 / 67.2   4 rows 84.5 / 71.3
-//   44.0 M (4096, 1536, 7)                     2 rows 58.7 / 64.6   3 rows 74.9 / 65.4   4 rows 94.7 / 73.0
-//   70.8 M (5120, 1536, 9)                     2 rows 83.7 / 79.5   3 rows 111 / 95.3    4 rows 143 / 108
-// Shapes without the split-K form (hidden or inter not a multiple of 512) keep the decode engine up to MOE_DECODE_ROWS.
-int moe_decode_rows(int hidden, int inter, int slots) {
-    if (hidden % 512 || inter % 512) return MOE_DECODE_ROWS;
-    const int64_t n = (int64_t)90000000 / ((int64_t)hidden * inter * slots);
-    return n < 1 ? 1 : n > MOE_DECODE_ROWS ? MOE_DECODE_ROWS : (int)n;
-}
-}  // namespace
-extern "C" {
 int gfr_moe_create(gfr_moe** out, int hidden, int inter, int routed, int topk, int max_rows) {
     return gfr_moe_create_shared(out, hidden, inter, routed, topk, max_rows, 1);
 }
@@ -451,11 +430,18 @@ int gfr_moe_create_shared(gfr_moe** out, int hidden, int inter, int routed, int 
     if (routed <= 0 || routed > 1023) return fail(GFR_EINVAL, "routed experts %d outside 1..1023", routed);
     if (topk <= 0 || topk > 31 || topk > routed) return fail(GFR_EINVAL, "topk %d", topk);
     if (max_rows <= 0 || max_rows > (1 << 16)) return fail(GFR_EINVAL, "max_rows %d", max_rows);
-    // decode engine for up to 64 rows; by default it takes the windows it wins (moe_decode_rows), the prefill engine
-    // (split-K MFMA for small windows) the rest
-    const int dec_rows = moe_decode_rows(hidden, inter, topk + 1);
+    // Decode engine for up to 64 rows; by default it takes windows of at most MOE_DECODE_ROWS rows at every layer, the
+    // prefill engine (split-K MFMA for small windows) the rest. At hidden 2048 (top-4, K = 4) the decode engine is the
+    // faster up to 4 rows, at wide layers up to 1 or 2 (us a layer, decode / prefill engine, Zipf(1.1), K = 4):
+    //   hidden 2048, inter 1536, 5 slots               3 rows 41.1 / 44.8   4 rows 50.9 / 52.9   5 rows 60.6 / 52.9
+    //   hidden 4096, inter 512, 9 slots, 288 experts   3 rows 54.8 / 64.9   4 rows 65.5 / 64.9   5 rows 85.6 / 67.0
+    //   hidden 4096, inter 1536, 7 slots               2 rows 58.7 / 64.6   3 rows 74.9 / 65.4   4 rows 94.7 / 73.0
+    //   hidden 5120, inter 1536, 9 slots               2 rows 83.7 / 79.5   3 rows 111 / 95.3    4 rows 143 / 108
+    // The engines multiply different weights (the decode engine the unrounded sums of the codebook's halves, the prefill
+    // engine their fp16 roundings), so the border is the caller's to move (gfr_moe_set_decode_rows), not the width's.
+    constexpr int MOE_DECODE_ROWS = 4;
     const int dec_cap = 64 < max_rows ? 64 : max_rows;
-    gfr_moe* m = new gfr_moe{hidden, inter, routed, topk, topk + 1, max_rows, dec_rows < max_rows ? dec_rows : max_rows,
+    gfr_moe* m = new gfr_moe{hidden, inter, routed, topk, topk + 1, max_rows,
                              MOE_DECODE_ROWS < max_rows ? MOE_DECODE_ROWS : max_rows,
                              nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1.f,
                              shared_exl3 ? 1 : 0, nullptr, 0, nullptr, nullptr};
@@ -492,10 +478,10 @@ int gfr_moe_set_decode_rows(gfr_moe* m, int decode_rows) {
     if (!m) return fail(GFR_EINVAL, "null moe");
     if (decode_rows < 0 || decode_rows > m->dec->max_rows || decode_rows > m->group_dec->max_rows)
         return fail(GFR_EINVAL, "decode_rows %d outside 0..%d", decode_rows, m->dec->max_rows);
-    if (decode_rows < m->max_rows && (!m->pre || m->max_rows <= MOE_DECODE_ROWS))
+    if (decode_rows < m->max_rows && !m->pre)
         return fail(GFR_EINVAL, "decode_rows %d leaves rows for the prefill engine, which this layer lacks",
                     decode_rows);
-    m->decode_rows = m->decode_most = decode_rows;
+    m->decode_rows = decode_rows;
     return 0;
 }
 
@@ -520,7 +506,7 @@ int moe_run(gfr_moe* m, hipStream_t stream, const gfr_exl3_experts* w, const uin
                     shared_stride);
     if (shared_ready && !shared) return fail(GFR_EINVAL, "a shared-ready event without a shared output");
     hipError_t e;
-    if (rows <= m->decode_rows || (rows <= m->decode_most && !gfr::prefill_fits(m->pre, w, rows))) {
+    if (rows <= m->decode_rows) {
         gfr_grouping* g = m->group_dec;
         if (rows == 1) {
             // three launches: gate/up (+ route, rotation), down (+ gate/up epilogue), down epilogue (+ combine)

@@ -140,8 +140,9 @@ float* gfr_moe_weights(const gfr_moe* m);        /* [rows][topk + 1] */
  * the prefill engine (windows above decode_rows), [rows * (topk + 1)][hidden] fp16 in the same pair order, matrix 0
  * (gate) or 1 (up). Windows of at most 256 rows rotate them in the grouping's launch. Null for mat not 0 or 1. */
 uint16_t* gfr_moe_rotated(const gfr_moe* m, int mat);
-/* Windows of at most decode_rows rows run the decode engine (at most 64; default 4, fewer where hidden x inter x
- * (topk + 1) passes 22 million weights, 1 from 45 million on), larger ones the prefill engine.
+/* Windows of at most decode_rows rows run the decode engine (default 4, at most 64), larger ones the prefill engine.
+ * A layer made for at most 4 rows has no prefill engine: values below max_rows are refused. Wide layers run 3 and 4 rows
+ * faster on the prefill engine (measured at K = 4 from hidden x inter x (topk + 1) = 44 million weights on).
  * rows == 1 runs three launches: gate/up GEMV (router and input rotation fused), down GEMV (gate/up epilogue fused),
  * sum of the down parts + combine. */
 int gfr_moe_set_decode_rows(gfr_moe* m, int decode_rows);

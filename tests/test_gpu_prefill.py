@@ -378,28 +378,37 @@ def test_split_windows_do_not_depend_on_the_window(gfr, bits):
         assert diff == 0, f"{diff} of {n} rows differ between a window of {n} rows and windows of 9"
 
 
-@pytest.mark.parametrize("hidden,inter,topk,limit", [(2560, 1536, 7, 2), (5120, 1536, 8, 1), (3072, 1536, 4, 3),
-                                                     (2048, 1536, 4, 4), (2560, 768, 7, 4)])
-def test_moe_small_windows_on_both_engines(gfr, oracle, hidden, inter, topk, limit):
-    """Windows on both sides of the engines' default border (from hidden x inter x slots): the prefill engine rotates its
-    rows, the decode engine leaves that probe alone; both give every token's output. A layer of at most 4 rows takes no
-    smaller border."""
+@pytest.mark.parametrize("bits", [2, 3, 4, 5])
+@pytest.mark.parametrize("hidden,inter,topk", [(2048, 1536, 4), (2560, 768, 7), (5120, 1536, 8)])
+def test_moe_small_windows_on_the_default_engine(gfr, oracle, hidden, inter, topk, bits):
+    """The default border is 4 rows at every width and bit width: windows of 1 to 4 rows run the decode engine (the
+    prefill engine's rotated rows, a probe, stay untouched), and the windows of 2 to 4 give every token the same bytes as a
+    window of two of it; 5 rows run the prefill engine. A layer of at most 4 rows has no prefill engine to leave rows for."""
     import synth
-    E, bits = topk + 2, 4
+    E = topk + 2
     w = synth.experts(E + 1, hidden, inter, bits, seed=800 + topk)
     m = gfr.Moe(hidden, inter, E, topk, 5)
     for rows in range(1, 6):
         x, lg = synth.activations(rows, hidden, 810 + rows), synth.zipf_logits(rows, E, topk, 1.1, 820 + rows)
+        pairs = []
+        for r in range(rows):
+            m.run(w, x[[r, r]].contiguous(), lg[[r, r]].contiguous(), 2)
+            pairs.append(m.output[:1].clone())
         for mat in (0, 1):
-            m.rotated(mat, rows).zero_()
+            m.rotated(mat, 5).zero_()
         m.run(w, x, lg, rows)
         torch.cuda.synchronize()
-        assert bool((m.rotated(0, rows) != 0).any()) == (rows > limit), rows
+        got = m.output[:rows].clone()
+        prefill = bool((m.rotated(0, 5) != 0).any())
+        assert prefill == (rows == 5), rows
+        if 1 < rows < 5:
+            assert torch.equal(got, torch.cat(pairs)), rows
         p, wt = oracle.route(lg.cpu().numpy(), topk, E)
         y = window_reference(oracle, w, x, p)
         want = np.einsum("rs,rsd->rd", wt.astype(np.float64), y.astype(np.float64))
         # the decode engine multiplies unrounded codebook sums (within 1e-2 of the reference's fp16 weights)
-        assert_rows_close(m.output[:rows].cpu().numpy(), want, rel_rms=1e-2 if rows <= limit else 2e-3, what=f"{rows} rows")
+        assert_rows_close(got.cpu().numpy(), want, rel_rms=2e-3 if prefill else 1e-2, what=f"{rows} rows")
     small = gfr.Moe(hidden, inter, E, topk, 3)
-    with pytest.raises(gfr.GfrError):
-        small.set_decode_rows(0)
+    small.set_decode_rows(3)
+    with pytest.raises(gfr.GfrError, match="lacks"):
+        small.set_decode_rows(2)
