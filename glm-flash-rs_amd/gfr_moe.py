@@ -133,12 +133,17 @@ def _ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
-# The current stream's handle without a torch.cuda.Stream object around it: every run call asks for it.
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# The current stream's handle without a torch.cuda.Stream object around it: every run call asks for it. None on a torch
+# without GPU support, where the host-only functions still work.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(stream=None) -> int:
-    return stream.cuda_stream if stream is not None else _raw_stream(torch.cuda.current_device())
+    if stream is None:
+        if _raw_stream is not None:
+            return _raw_stream(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
+    return stream.cuda_stream
 
 
 class _DeviceArray:
