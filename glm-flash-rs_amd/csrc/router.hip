@@ -132,8 +132,27 @@ __global__ void __launch_bounds__(256) router_logits_kernel(const uint16_t* __re
 // L2 (a row is read by E / (16 EB) workgroups, an expert by rows / (16 RB)), so the tiles are as large as the registers
 // allow (RB x EB = 4 x 5: two sums of 80 and 72 of loads) and one round of workgroups covers the window. Measured against
 // router_logits_kernel (us): 4096 rows, hidden 4096, 288 experts 202 -> 38; 8192 rows, hidden 5120, 160 experts 599 ->
-// 48; 700 rows 60 -> 15; 128 rows, 288 experts 12.9 -> 12.7; below that the dot products win (64 rows 9.6 against 12.6).
+// 48; 700 rows 60 -> 15. Error against fp64 at hidden 1024, 2048, 5120, 16384 and 65536: 6.5, 7.0, 7.9, 10.1 and 16.1e-8,
+// 6.8, 7.4, 8.7, 12.3 and 24.6e-8 for the dot products.
+//
+// Which form a window runs: a wave of this kernel waits for a round of loads every 1024 k (hidden / 1024 rounds of about
+// 2.5 us), while the dot products take one pass of 4096 k and grow with their programs (8 experts x 8 rows, four waves).
+// Measured (us, dot products / matrix core):
+//   one program a CU (rows x experts = 16384: 64 experts, 256 rows): hidden 1024 7.1 / 4.9, 1792 7.2 / 6.9, 2048 7.3 / 7.5,
+//     3072 8.1 / 10.2, 4096 8.6 / 12.8, 5120 18.2 / 16.0, 6144 18.2 / 18.0, 8192 22.1 / 23.1, 16384 40.2 / 43.7
+//   1.25 a CU (160 experts, 128 rows): 2048 8.5 / 7.6, 2560 8.9 / 9.1, 3072 9.3 / 10.2, 4096 9.9 / 12.8
+//   two a CU (64 experts, 512 rows): 2048 8.5 / 7.5, 2560 9.0 / 9.1, 3072 9.5 / 10.2, 4096 11.2 / 12.7
+//   2.5 a CU (160 experts, 256 rows): 4096 12.7 / 12.8; above that, and below 1792 at any count, the matrix core wins
+// Above one program a CU the dot products win only at hidden sizes that are multiples of 512 (4088, 96 experts, 256 rows
+// 10.0 / 8.8): there the 16 rows of a fragment lie a multiple of 1 KB apart, so that its loads likely meet in few of the
+// L2's channels.
 constexpr int ROUTER_MFMA_ROWS = 128;
+static bool router_on_mfma(int rows, int E, int D) {
+    if (rows < ROUTER_MFMA_ROWS) return false;
+    const int64_t products = (int64_t)rows * E;
+    if (products <= 16384) return D <= 1792 || (D > 4096 && D < 6144);
+    return products > 32768 || D < 2560 || D > 4096 || D % 512;
+}
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 constexpr int ROUTER_WAVES = 8;
@@ -243,7 +262,7 @@ int router_logits_max_hidden() { return 1 << 16; }
 
 hipError_t launch_router_logits(hipStream_t s, const uint16_t* x, int x_stride, const uint16_t* W, int D, int E,
                                 int rows, float* logits) {
-    if (rows >= ROUTER_MFMA_ROWS) {
+    if (router_on_mfma(rows, E, D)) {
         // the tile with the lowest estimate: rounds of one workgroup a CU, each as long as its operand reads (rows and
         // experts of a tile) plus a fixed part
         const auto wgs = [&](int rb, int eb) { return (rows + 16 * rb - 1) / (16 * rb) * ((E + 16 * eb - 1) / (16 * eb)); };

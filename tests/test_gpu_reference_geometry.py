@@ -115,6 +115,21 @@ def test_router_logits_matrix_tiles(gfr, rows, routed, hidden):
     assert ((got - want).abs() <= (hidden / 256 + 12) * 2.0 ** -24 * mag).all()
 
 
+@pytest.mark.parametrize("rows,routed,hidden,dots", [
+    (128, 128, 2048, True), (129, 128, 2048, False),      # one program of the dot products a CU, and more
+    (256, 64, 4096, True), (256, 64, 1792, False), (256, 64, 5120, False), (128, 32, 8192, True),
+    (128, 160, 3072, True), (128, 160, 3080, False), (128, 160, 2048, False),   # up to two: multiples of 512
+    (512, 64, 4096, True), (513, 64, 4096, False)])
+def test_router_logits_form_of_small_products(gfr, rows, routed, hidden, dots):
+    """Windows of 128 rows and more whose dot products are few programs keep them: the bytes are those of windows of 127
+    rows, which always run them. The others run the matrix core, whose sums are in another order."""
+    g = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    x = torch.randn((rows, hidden), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((routed, hidden), generator=g, device="cuda").to(torch.bfloat16)
+    got = gfr.router_logits(x, w)
+    small = torch.cat([gfr.router_logits(x[r:r + 127].contiguous(), w) for r in range(0, rows, 127)])
+    assert torch.equal(got, small) == dots
+
 
 @pytest.mark.parametrize("rows", [1, 3, 40, 300])
 def test_moe_reference_layout_shared_output(gfr, oracle, weights, rows):
