@@ -724,7 +724,8 @@ def moe_token_static(w: Exl3Experts, routed: int, topk: int, input: torch.Tensor
 
 
 def router_logits(input: torch.Tensor, router_weight: torch.Tensor, stream=None) -> torch.Tensor:
-    """gfr_router_logits: [rows, routed] fp32 logits of bf16 rows [rows, hidden] and a bf16 weight [routed, hidden]."""
+    """gfr_router_logits: [rows, routed] fp32 logits of bf16 rows [rows, hidden] and a bf16 weight [routed, hidden].
+    From 128 rows on the sums may be taken in another order (on the matrix core) than in smaller windows."""
     if input.dtype != torch.bfloat16 or router_weight.dtype != torch.bfloat16:
         raise ValueError("router logits take bf16 rows and a bf16 weight")
     rows, hidden = input.shape

@@ -226,7 +226,11 @@ int gfr_route_topk_biased(hipStream_t stream, const float* logits, const float* 
 int gfr_route_topk(hipStream_t stream, const float* logits, int rows, int routed, int topk, int32_t* picks,
                    float* weights);
 /* Router logits (moe.rs:77-87, router_part [1,9,8] + router_sum; Triton, source absent): logits[r][e] =
- * sum over k of input[r][k] * router_weight[e][k], bf16 inputs, fp32 products and sums in a fixed order.
+ * sum over k of input[r][k] * router_weight[e][k], bf16 inputs. Two forms, each with a summation order of its own that
+ * nothing else changes: fp32 dot products in windows of up to 127 rows, and in larger ones with few rows x experts; on
+ * the matrix core in the others (fp32 chains of 128 k, added in fp32 over an eighth of the hidden size, the eighths in
+ * fp64, rounded once). A row's logits may differ between the forms in their last bits, within either one's rounding
+ * error, and picks of nearly equal logits with them.
  * input [rows][input_stride] bf16, router_weight [routed][hidden] bf16, logits [rows][routed] fp32; hidden a
  * multiple of 8, at most 65536; input_stride a multiple of 8, input and router_weight 16-byte aligned (rows are read
  * 16 bytes at a time). */

@@ -131,6 +131,21 @@ def test_router_logits_form_of_small_products(gfr, rows, routed, hidden, dots):
     assert torch.equal(got, small) == dots
 
 
+def test_router_logits_of_one_row_in_both_forms(gfr):
+    """The same rows in windows of 127 (dot products) and of 128 (the matrix core at 288 experts): a logit differs by no
+    more than both forms' rounding: (hidden / 256 + 12) roundings of 2^-24 of the sum of the products' magnitudes on the
+    matrix core, and (hidden / 64 + 7) for the dot products (a lane's hidden / 64 products in pairs, each pair at most two
+    roundings, and the tree of 64 lanes)."""
+    hidden, routed = 4096, 288
+    g = torch.Generator(device="cuda").manual_seed(127)
+    x = torch.randn((128, hidden), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((routed, hidden), generator=g, device="cuda").to(torch.bfloat16)
+    small, large = gfr.router_logits(x[:127].contiguous(), w).double(), gfr.router_logits(x, w)[:127].double()
+    assert not torch.equal(small, large)
+    mag = x[:127].double().abs() @ w.double().abs().t()
+    assert ((small - large).abs() <= (hidden / 256 + 12 + hidden / 64 + 7) * 2.0 ** -24 * mag).all()
+
+
 @pytest.mark.parametrize("rows", [1, 3, 40, 300])
 def test_moe_reference_layout_shared_output(gfr, oracle, weights, rows):
     """Moe::run_prefetched at the reference's layout (moe.rs:77-181): router logits from the hidden rows, GLM's gate
