@@ -361,7 +361,7 @@ __global__ void __launch_bounds__(256) prefill_rot2_kernel(const uint16_t* __res
 }
 
 // The layer's FP8 shared expert in a window of at most 16 rows: its gate/up programs (8 intermediate indices a
-// workgroup of 8 waves, one K slice each) are workgroups 1 .. inter / 8 of the launches below, which need nothing of each
+// workgroup of 8 waves, one K slice each) are workgroups 1 .. inter / 8 of the launch below, which need nothing of each
 // other; its down programs ride on the gate/up epilogue's launch. Its own two launches took 8.0 + 4.0 us next to these
 // launches' 12.6 and 4.7 (12 rows, 288 experts): a layer 93 -> 85 us.
 __device__ __forceinline__ void fp8_gu_workgroup(const Fp8Args& f, int rows) {
@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(512) route_group_rot_kernel(const float* __res
 // group_small_kernel's work (with the item plan) in workgroup 0 and the rotation's tasks in the others, for windows
 // whose picks are routed: launch_route_group_rot's second launch where one workgroup's routing of every row would
 // outlast the rest.
-template <int MATS, bool FP8>
+template <int MATS>
 __global__ void __launch_bounds__(512) group_small_rot_kernel(const int* __restrict__ picks, int rows, int slots, int E,
                                                               int* __restrict__ ids, int* __restrict__ count,
                                                               int* __restrict__ members, int maxm, int bm,
@@ -425,7 +425,7 @@ __global__ void __launch_bounds__(512) group_small_rot_kernel(const int* __restr
                                                               const uint16_t* __restrict__ suh0,
                                                               const uint16_t* __restrict__ suh1,
                                                               uint16_t* __restrict__ out0, uint16_t* __restrict__ out1,
-                                                              int K, int exl3_slots, const Fp8Args f) {
+                                                              int K, int exl3_slots) {
     extern __shared__ uint32_t lds[];
     __shared__ __attribute__((aligned(16))) int scan_scratch[16];
     if (blockIdx.x == 0) {
@@ -437,9 +437,7 @@ __global__ void __launch_bounds__(512) group_small_rot_kernel(const int* __restr
         return;
     }
     const int lane = threadIdx.x & 63;
-    const int fwg = FP8 ? f.inter / 8 : 0;
-    if (FP8 && (int)blockIdx.x <= fwg) return fp8_gu_workgroup(f, rows);
-    const int task = ((int)blockIdx.x - 1 - fwg) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int task = (blockIdx.x - 1) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int KP = K / 256, row = task / KP, bp = task % KP;
     if (row >= rows) return;
     rot2_task<MATS>(x, x_stride, [&] { return lane < exl3_slots ? picks[row * slots + lane] : 0; }, suh0, suh1, out0,
@@ -1256,11 +1254,14 @@ static bool fused_window(const gfr_fast_experts* fx, const gfr_exl3_experts* w, 
            route_group_lds(rows, topk + 1, routed + 1) <= GROUP_LDS_MAX && (d.hidden / 128) % 2 == 0 && w->bits >= 2 &&
            w->bits <= 5;
 }
+constexpr int FP8_ROWS = 16;              // one tile of the FP8 programs
 bool prefill_takes_fp8(const gfr_fast_experts* fx, const gfr_exl3_experts* w, int rows, int routed, int topk) {
-    return rows <= 16 && fused_window(fx, w, rows, routed, topk) && window_form(fx, rows) == Form::SPLIT &&
+    return rows <= FP8_ROWS && fused_window(fx, w, rows, routed, topk) && window_form(fx, rows) == Form::SPLIT &&
            route_group_lds(rows, topk + 1, routed + 1) + sizeof(Fp8Part) <= GROUP_LDS_MAX;
 }
-constexpr int ROUTE_ONE_PICKS = 100;   // picks of a window up to which one launch routes, groups and rotates it
+// Windows of up to this many rows, or of up to this many picks, are routed, grouped and rotated by one launch.
+constexpr int ROUTE_ONE_ROWS = 16, ROUTE_ONE_PICKS = 100;
+static_assert(FP8_ROWS <= ROUTE_ONE_ROWS, "the FP8 shared expert rides on the one launch");
 hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr_exl3_experts* w,
                                   const uint16_t* input, int input_stride, const float* logits, int rows, int routed,
                                   int topk, int* picks, float* weights, int* ids, int* count, int* members, int maxm,
@@ -1273,19 +1274,21 @@ hipError_t launch_route_group_rot(gfr_fast_experts* fx, hipStream_t s, const gfr
     if (fp8) f = Fp8Args{fp8->gu_w, fp8->gu_s, input, fp8->gu, fp8->act, nullptr, fp8->hidden, fp8->inter};
     constexpr int WG = 512;                              // route_group measured the same at 512 and 1024 threads
     const int tasks = rows * (d.hidden / 256), grid = 1 + (fp8 ? f.inter / 8 : 0) + (tasks + WG / 64 - 1) / (WG / 64);
-    // Workgroup 0's eight waves route the rows eight at a time, 0.14 us a row at top-4 of 64, 0.27 at top-8 of 160 and
-    // 0.53 at GLM's top-8 of 288: past about 100 picks a launch that routes every row at once, ahead of the grouping and
-    // the rotation, costs less. A layer, one launch / two (us): hidden 2048, top-4 of 64: 20 rows 73.9 / 75.0, 32 rows
-    // 89.6 / 88.8, 100 rows 137 / 128, 220 rows 187 / 171; hidden 5120, top-8 of 160: 20 rows 254.6 / 255.3, 77 rows 501 /
-    // 494, 220 rows 680 / 638; hidden 4096, top-8 of 288: 20 rows 129 / 124, 100 rows 270 / 235, 220 rows 416 / 336.
-    if (rows * topk > ROUTE_ONE_PICKS) {
+    // Workgroup 0's eight waves route the rows eight at a time, 1.1 us a round at top-4 of 64 experts, 2.2 at top-8 of 160
+    // and 4.2 at GLM's top-8 of 288 (partly behind the rotation and the FP8 programs): past two rounds and about 100 picks
+    // a launch that routes every row at once, ahead of the grouping and the rotation, costs no more. A layer, one launch /
+    // two (us, K = 4, graph replays): hidden 2048, top-4 of 64: 16 rows 65.2 / 66.4, 24 rows 79.8 / 79.8, 26 rows 80.4 /
+    // 80.0, 32 rows 81.7 / 80.7, 48 rows 98.4 / 96.7; hidden 5120, top-8 of 160: 13 rows 187.5 / 188.6, 16 rows 213.7 /
+    // 214.6, 20 rows 232.2 / 232.1, 32 rows 285.9 / 283.4, 48 rows 404 / 402; hidden 4096, top-8 of 288, FP8 shared
+    // expert: 14 rows 84.1 / 84.4, 16 rows 96.3 / 96.3, 20 rows 122.9 / 119.1, 32 rows 155 / 148, 48 rows 193 / 179;
+    // 220 rows (eager) 187 / 171, 680 / 638 and 416 / 336.
+    if (rows > ROUTE_ONE_ROWS && rows * topk > ROUTE_ONE_PICKS) {
         hipError_t e = launch_route(s, logits, rows, routed, topk, routed, picks, weights, bias, scale);
         if (e != hipSuccess) return e;
-        auto go = fp8 ? group_small_rot_kernel<2, true> : group_small_rot_kernel<2, false>;
-        go<<<grid, WG, group_small_lds(rows, slots, routed + 1), s>>>(
+        group_small_rot_kernel<2><<<grid, WG, group_small_lds(rows, slots, routed + 1), s>>>(
             picks, rows, slots, routed + 1, ids, count, members, maxm, prefill_item_rows(fx, rows, w->bits), fx->ucnt,
             fx->items, fx->plan, w->experts, input, input_stride, w->suh_g, w->suh_u, fx->xg, fx->xu, d.hidden,
-            d.exl3_slots, f);
+            d.exl3_slots);
         return hipGetLastError();
     }
     auto go = fp8 ? route_group_rot_kernel<2, true> : route_group_rot_kernel<2, false>;

@@ -116,3 +116,18 @@ def assert_rows_close(got, want, rel_rms=1e-3, rel_max=1e-2, what=""):
     assert rms[worst] < rel_rms and mx < rel_max, \
         f"{what}: worst row {worst} relative RMS {rms[worst]:.3g} (median {np.median(rms):.3g}), max {mx:.3g}"
     return float(rms[worst]), float(mx)
+
+
+def graph_kernels(run) -> int:
+    """The launches of run(stream), counted as the nodes of a graph captured from it."""
+    import ctypes
+    import re
+    run(torch.cuda.current_stream())                     # every kernel loaded before the capture
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=stream):
+        run(stream)
+    hip = ctypes.CDLL(re.search(r"\S*/libamdhip64\.so\S*", open("/proc/self/maps").read())[0])
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value

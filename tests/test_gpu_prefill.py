@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from refs import DecodedExperts, assert_close, assert_rows_close, np_u16, window_reference
+from refs import DecodedExperts, assert_close, assert_rows_close, graph_kernels, np_u16, window_reference
 
 pytestmark = pytest.mark.gpu
 
@@ -219,8 +219,12 @@ def test_prefill_rotation_bitexact(gfr, oracle, hidden, slots, rows, shared_x):
 @pytest.mark.parametrize("hidden,routed,topk,rows,glm", [
     (2048, 64, 4, 37, False),     # config 3's shape: softmax gate, 5 slots
     (1024, 288, 8, 9, True),      # the reference's router: GLM's biased sigmoid gate over 288 experts, 9 slots
-    (1024, 288, 8, 12, True),     # 96 picks: the most one launch routes, groups and rotates ...
-    (1024, 288, 8, 13, True),     # ... 104: a launch that routes, then one that groups and rotates
+    (1024, 288, 8, 12, True),     # 96 picks
+    (1024, 288, 8, 13, True),     # ... and 104, in two rounds of eight rows
+    (1024, 288, 8, 16, True),     # the most rows above 100 picks that one launch routes, groups and rotates ...
+    (1024, 288, 8, 17, True),     # ... a launch that routes, then one that groups and rotates
+    (1024, 64, 4, 25, False),     # 100 picks: still one launch ...
+    (1024, 64, 4, 26, False),     # ... 104: two
     (512, 16, 2, 256, False),     # the largest window of those launches
     (512, 16, 2, 300, False),     # larger windows: the rotation rides on the grouping's scatter launch
     (1024, 288, 8, 260, True),    # ... with GLM's gate, full-K items
@@ -288,6 +292,19 @@ def test_moe_prefill_graph_replays(gfr, rows):
             graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(m.output[:rows], eager[1])
+
+
+@pytest.mark.parametrize("routed,topk,rows,launches", [
+    (160, 8, 12, 5), (160, 8, 13, 5), (288, 8, 16, 5), (288, 8, 17, 6), (64, 4, 25, 5), (64, 4, 26, 6), (64, 1, 100, 5),
+    (64, 1, 101, 6)])
+def test_window_launches(gfr, routed, topk, rows, launches):
+    """A window's launches: route + group + rotation, gate/up programs, their epilogue, down programs, finish; above 16
+    rows and 100 picks the routing is a launch of its own."""
+    import synth
+    w = synth.experts(routed + 1, 512, 512, 2, seed=30)
+    x, lg = synth.activations(rows, 512, 31), synth.logits(rows, routed, 32)
+    m = gfr.Moe(512, 512, routed, topk, rows)
+    assert graph_kernels(lambda s: m.run(w, x, lg, rows, stream=s)) == launches
 
 
 def test_split_window_with_many_experts(gfr, oracle):
