@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from refs import DecodedExperts, assert_close, assert_rows_close, np_u16
+from refs import DecodedExperts, assert_close, assert_rows_close, graph_kernels, np_u16
 
 pytestmark = pytest.mark.gpu
 
@@ -232,18 +232,23 @@ def test_moe_run_fp8_one_token_forms(gfr, oracle, routed, topk, H, I):
         assert torch.equal(m.output[:1], got)
 
 
-@pytest.mark.parametrize("routed,topk,H,I,rows", [
-    (16, 4, 512, 256, 5),        # 32 down tiles, two a grid column
-    (16, 4, 512, 768, 16),       # six a column: the last column's tail is idle; 16 rows: a full tile
-    (16, 4, 512, 768, 17),       # the first window past the tile: its own launches
-    (12, 4, 1024, 256, 1),       # one row through the prefill engine
-    (40, 8, 1024, 256, 12),      # 96 picks: one launch routes, groups and rotates
-    (40, 8, 1024, 256, 13),      # 104 picks: two
-    (1000, 4, 512, 256, 7)])     # many experts: the grouping's LDS next to the program's
-def test_moe_run_fp8_window_forms(gfr, routed, topk, H, I, rows):
-    """Windows of the prefill engine with the FP8 shared expert: up to 16 rows ride on the layer's launches. The bytes
-    are those of gfr_moe_run_shared fed with gfr_shared_fp8's output (the same programs: no tolerance), eagerly, on
-    another window after it, and in every replay of a captured graph."""
+@pytest.mark.parametrize("routed,topk,H,I,rows,rides", [
+    # hidden or inter not a multiple of 512, which the split-K programs need: the shared expert's own launches
+    (16, 4, 512, 256, 5, False), (16, 4, 512, 768, 16, False), (16, 4, 512, 768, 17, False), (12, 4, 1024, 256, 1, False),
+    (40, 8, 1024, 256, 12, False), (40, 8, 1024, 256, 13, False), (1000, 4, 512, 256, 7, False),
+    (16, 4, 512, 512, 5, True),       # 32 down tiles in 8 columns of 4 workgroups
+    (16, 4, 512, 1536, 16, True),     # in 3 columns of 12, the last four idle; 16 rows: a full tile
+    (16, 4, 512, 1536, 17, False),    # the first window past the tile
+    (12, 4, 1024, 512, 1, True),      # one row through the prefill engine
+    (40, 8, 1024, 512, 12, True),     # 96 picks ...
+    (40, 8, 1024, 512, 13, True),     # ... and 104
+    (288, 8, 4096, 512, 16, True),    # the served model's layer: a slice of 512 k a wave
+    (1000, 4, 512, 512, 7, True)])    # many experts: the grouping's LDS next to the program's
+def test_moe_run_fp8_window_forms(gfr, routed, topk, H, I, rows, rides):
+    """Windows of the prefill engine with the FP8 shared expert: up to 16 rows ride on the layer's launches at a shape
+    that has the split-K programs (two launches fewer, counted in the captured graph). The bytes are those of
+    gfr_moe_run_shared fed with gfr_shared_fp8's output (the same programs: no tolerance), eagerly, on another window
+    after it, and in every replay of a captured graph."""
     import synth
     w = synth.experts(routed, H, I, BITS, seed=routed)
     sw1 = synth.fp8_shared(H, I, seed=routed + 1)
@@ -263,6 +268,9 @@ def test_moe_run_fp8_window_forms(gfr, routed, topk, H, I, rows):
         want = m2.output[:rows].clone()
         assert torch.equal(m.shared_output[:rows], shared)
         assert torch.equal(m.output[:rows], want)
+    fp8 = graph_kernels(lambda st: m.run_fp8(w, x, lg, sw1, rows, stream=st))
+    given = graph_kernels(lambda st: m2.run(w, x, lg, rows, shared=shared, stream=st))
+    assert fp8 - given == (0 if rides else 2)
     s = torch.cuda.Stream()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(s):
