@@ -13,11 +13,11 @@
 //     (16 n x 8 k) once k is taken in the pair order of exl3_format.hpp (pair_row); the token rows (B operand) are
 //     staged in LDS in that same order, so no weight ever goes through LDS and none is decoded twice in a workgroup.
 //   * workgroup = 4 waves, a tile of BM member rows of one expert x 128 (gate/up: both matrices) or 256 (down)
-//     output columns, two workgroups a CU (three where items are short, see PF_FEW); each wave owns 64 columns x BM rows (4 BM / 16 MFMA 16x16 accumulators),
-//     K in steps of 32, multi-stage direct-to-LDS staging and a register pipeline (next step's decode during this
-//     step's MFMAs). BM = 176 for K = 4: the trellis decode (VALU) is amortised over more rows, an expert of 512
-//     members takes 3 passes instead of 4, and 244 VGPRs and two workgroups' stages (2 x 80.6 KB) still fit.
-//     K = 2, 3 and 5 decode their fragments directly as well (176, 160 and 144 rows, the most without spills).
+//     output columns, two workgroups a CU (three where items are short, see PF_FEW); each wave owns 64 columns x BM
+//     rows (4 BM / 16 MFMA 16x16 accumulators), K in steps of 32, multi-stage direct-to-LDS staging and a register
+//     pipeline (next step's decode during this step's MFMAs). BM = 176 for K = 4: the trellis decode (VALU) is amortised
+//     over more rows, an expert of 512 members takes 3 passes instead of 4, and two workgroups' stages (2 x 80.6 KB)
+//     still fit. K = 2, 3 and 5 decode their fragments directly as well (176, 160 and 144 rows).
 //   * the 128 columns of a gate/up item, and each 128 of a down item, are one Hadamard block, so the epilogue
 //     (transforms, scales, SwiGLU) runs in the workgroup: accumulators -> LDS (32 rows at a time) -> registers with
 //     8 consecutive values a lane and four rows a wave, so that three of the seven butterfly stages stay in registers.
@@ -34,9 +34,13 @@
 
 namespace gfr {
 
-// Member rows a full-K item at each width: the most that keep two workgroups' stages in LDS and the kernel within
-// 256 VGPRs without spills (K = 4: 244 VGPRs at 176 rows, 2 x 80.6 KB of LDS; K = 3 at 160 rows: 252; K = 5 at
-// 144: 256; K = 2 at 176: 239). Larger items decode each weight tile for more rows.
+// Member rows a full-K item at each width: the most whose two workgroups' stages fit the LDS (K = 4: 2 x 80.6 KB) and
+// whose full body alone fits 256 VGPRs (238, 252, 245 and 254 for gate/up at K = 2, 3, 4 and 5). Larger items decode each
+// weight tile for more rows. With the smaller bodies (below) the gate/up and down kernels take 256 and 256 VGPRs at K = 2
+// (1 and 5 more spilled, outside the blocks that hold the MFMAs), 256 and 256 at K = 3 (5 and 4 spilled), 256 and 242 at
+// K = 4, 246 and 217 at K = 5, among them lanes that keep up to 62 spilled SGPRs. A layer, one body and the fragment
+// decode of that time / now (us, uniform): 8192 rows, hidden 2048, K = 2 1174 / 1127, K = 3 1288 / 1233, K = 4 1148 /
+// 1139, K = 5 1327 / 1249.
 #ifndef PF_BM2_ROWS
 #define PF_BM2_ROWS 176
 #endif
@@ -57,9 +61,10 @@ constexpr int pf_bm_for(int bits) { return bits == 2 ? PF_BM2 : bits == 3 ? PF_B
 // its trellis in HBM needs. Measured against one body (us a layer): 4096 rows of the FP8-shared geometry (median 34 rows
 // an expert) 1250 -> 1208; 1500 rows, hidden 5120, K = 3 1504 -> 1453.
 constexpr int PF_SMALL = 32, PF_MID = 96;
-// Windows of few rows an expert run PF_FEW-row items on kernels small enough for three workgroups a CU (168 VGPRs,
-// 53 KB of LDS): their programs are bound by the trellis decode's VALU work next to the stage waits, which a third wave a
-// SIMD covers. See window_form for where this form is taken and what it measured.
+// Windows of few rows an expert run PF_FEW-row items on kernels small enough for three workgroups a CU (168 VGPRs, at most
+// 53 KB of LDS; the gate/up kernels spill 1, 14, 9 and 15 VGPRs at K = 2, 3, 4 and 5, the down kernels none): their
+// programs are bound by the trellis decode's VALU work next to the stage waits, which a third wave a SIMD covers. See
+// window_form for where this form is taken and what it measured.
 constexpr int PF_FEW = 96, PF_FEW_OCC = 3;
 constexpr int PF_MAXU = 1024;       // distinct experts a window (grid / plan bound)
 
