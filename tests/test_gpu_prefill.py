@@ -120,8 +120,7 @@ def test_moe_prefill_config4_tokens(gfr, oracle):
 @pytest.mark.parametrize("rows", [40, 320])
 def test_fast_experts_bit_widths(gfr, oracle, bits, rows):
     """K = 2, 3, 4, 5 (config 5's mixed bit rates) at C5's hidden size against the oracle: every width decodes its
-    trellis straight into MFMA A fragments (K = 4 from word pairs, the others through one funnel shift a group of four
-    values). 40 rows (360 pairs) run the split-K programs, 320 rows (2880 pairs) the full-K items with the fused
+    trellis straight into MFMA A fragments, through one funnel shift a group of four values. 40 rows (360 pairs) run the split-K programs, 320 rows (2880 pairs) the full-K items with the fused
     epilogues."""
     import synth
     Dk, Nk, E, slots, maxm = 5120, 1536, 9, 9, rows
@@ -262,13 +261,15 @@ def test_moe_fused_rotation_bitexact(gfr, oracle, hidden, routed, topk, rows, gl
                     f"matrix {mat} row {r} slot {s}: {np.sum(got[r * (topk + 1) + s] != want)} values differ"
 
 
+@pytest.mark.parametrize("N,bits", [(512, 4), (256, 4), (256, 3)])
 @pytest.mark.parametrize("rows", [32, 300, 1024])
-def test_moe_prefill_graph_replays(gfr, rows):
+def test_moe_prefill_graph_replays(gfr, rows, N, bits):
     """A captured prefill-engine layer replays to the eager bytes, across two weight sets and routings: a small window
-    (route + group + rotation in one launch, split-K programs), a larger split-K window (the rotation in the
-    grouping's scatter launch) and a full-K window. Each replay follows eager work that clears the output."""
+    (route + group + rotation in one launch), a larger one (the rotation in the grouping's scatter launch), both on the
+    split-K programs at inter 512 and on the few-row items at 256, which has no split-K form, and a window on the largest
+    items. Each replay follows eager work that clears the output."""
     import synth
-    E, D, N, bits, topk = 16, 512, 256, 4, 2
+    E, D, topk = 16, 512, 2
     ws = [synth.experts(E + 1, D, N, bits, seed=s) for s in (31, 32)]
     xs = [synth.activations(rows, D, 33 + j) for j in range(2)]
     lgs = [synth.logits(rows, E, 35 + j) for j in range(2)]
